@@ -191,14 +191,8 @@ struct State {
     int ndev = 0;
     int rank = 0;
     hipStream_t st = nullptr;
-    hipEvent_t ev_send = nullptr, ev_jp = nullptr, ev_desc = nullptr;
-    bool ev_send_live = false, ev_jp_live = false, ev_desc_live = false;
-    HostBuf<ClusterDesc> h_desc;
-    DevBuf<ClusterDesc> d_desc;
-    // What d_desc holds (uploaded by enqueue_regf); an unchanged table is not
-    // uploaded again.
-    std::vector<ClusterDesc> desc_up;
-
+    hipEvent_t ev_send = nullptr, ev_jp = nullptr;
+    bool ev_send_live = false, ev_jp_live = false;
     int nbmax = 0;
     int nj = 0;       // current j count used by regf
     int njp = 0;      // j slots covered by the predictor state
@@ -357,7 +351,6 @@ void devinit(int irank) {
     HIPCHK(hipEventCreateWithFlags(&S.ev_p2end, hipEventDisableTiming));
     HIPCHK(hipEventCreateWithFlags(&S.ev_send, hipEventDisableTiming));
     HIPCHK(hipEventCreateWithFlags(&S.ev_jp, hipEventDisableTiming));
-    HIPCHK(hipEventCreateWithFlags(&S.ev_desc, hipEventDisableTiming));
     S.jst.ensure(1);
     S.err.ensure(1);
     S.h_err.ensure(1);
@@ -422,9 +415,8 @@ int pick_group() {
     const char *g = getenv("GPUNB_REGF_GROUP");
     if (g && atoi(g) == 2) return 2;
     if (g && atoi(g) == 4) return 4;
-    // Two pairs per group: the mixed kernel fits 4 resident waves per SIMD
-    // and the FP64 kernel 5 (four pairs: more than 128 VGPRs, 3 waves),
-    // which hides the latency of the dependent chains better.
+    // Two pairs per group: five resident wavefronts per SIMD (four pairs:
+    // three), which hides the latency of the dependent chains better.
     return 2;
 }
 
@@ -464,13 +456,20 @@ int resident_waves(int m_flag, int group, int prec) {
 
 // j slices per i-wavefront: enough wavefronts (kP1W per slice task) to
 // fill the resident capacity `rounds` times; a slice holds at least one
-// tile per wavefront where the j set allows.
-int decompose(int ni_c, int ntile, int m_flag, int group, int prec) {
+// tile per wavefront where the j set allows.  Slices are cut in units of
+// 2^ju j: whole tiles for the mixed kernel, 16 j for the FP64 kernel, whose
+// loop has no work per tile, so that the wavefronts of a launch get equal
+// shares.  FP64 launches that would leave SIMDs without a wavefront at one
+// tile each take slices down to one unit per wavefront.
+int decompose(int ni_c, int ntile, int m_flag, int group, int prec, int &ju) {
     const int n_iw = cdiv(ni_c, 64);
     const double target = resident_waves(m_flag, group, prec) * pick_rounds(ni_c);
+    ju = prec >= 64 ? 4 : 6;
+    const bool fine = prec >= 64 && (long long)n_iw * ntile < 1024;
+    const int nu = fine ? ntile << (6 - ju) : ntile;
     int ns = (int)std::lround(target / ((double)n_iw * kP1W));
     ns = std::max(ns, 1);
-    ns = std::min(ns, std::max(ntile / kP1W, 1));
+    ns = std::min(ns, std::max(nu / kP1W, 1));
     return ns;
 }
 
@@ -599,7 +598,9 @@ void enqueue_regf(int ni, const double *xi, const double *vi, const double *h2,
     for (int c = 0; c < nch; ++c) {
         const int c0 = c * chunk;
         const int nc = std::min(chunk, ni - c0);
-        const int ns = ntile == 0 ? 1 : decompose(nc, ntile, m_flag, group, prec);
+        int ju = 6;
+        const int ns =
+            ntile == 0 ? 1 : decompose(nc, ntile, m_flag, group, prec, ju);
         const int cap = std::max(nnbmax, 1);
         ensure_regf_scratch(nc, ns, cap, c & 1);
         ClusterDesc &D = nd[c];
@@ -610,23 +611,9 @@ void enqueue_regf(int ni, const double *xi, const double *vi, const double *h2,
         D.ni = nc;
         D.n_iw = cdiv(nc, 64);
         D.nslice = ns;
+        D.ju = ju;
         D.cap = cap;
         D.ipb = pass2_ipb(nc);
-    }
-    const size_t had = S.d_desc.n;
-    S.d_desc.ensure((size_t)nch);
-    if (S.d_desc.n != had) S.desc_up.clear();   // new buffer: nothing held
-    if (S.desc_up.size() != nd.size() ||
-        memcmp(S.desc_up.data(), nd.data(), nd.size() * sizeof(ClusterDesc))) {
-        // h_desc may still be read by the previous upload.
-        wait_event(S.ev_desc, S.ev_desc_live);
-        S.h_desc.ensure((size_t)nch);
-        memcpy(S.h_desc.p, nd.data(), nd.size() * sizeof(ClusterDesc));
-        HIPCHK(hipMemcpyAsync(S.d_desc.p, S.h_desc.p, nch * sizeof(ClusterDesc),
-                              hipMemcpyHostToDevice, S.st));
-        HIPCHK(hipEventRecord(S.ev_desc, S.st));
-        S.ev_desc_live = true;
-        S.desc_up = nd;
     }
     for (int c = 0; c < nch; ++c) {
         const ClusterDesc &D = nd[c];
@@ -657,7 +644,7 @@ void enqueue_regf(int ni, const double *xi, const double *vi, const double *h2,
         L.group = group;
         L.prec = prec;
         L.err = S.err.p;
-        L.desc = S.d_desc.p + c;
+        L.one = D;
         L.ncl = 1;
         L.ntask = (long long)D.n_iw * D.nslice;
         L.nblk2 = cdiv(D.ni, D.ipb);
@@ -716,14 +703,15 @@ void enqueue_regf_noalloc(int ni, const double *xi, const double *vi,
     const int cap = std::max(nnbmax, 1);
     const size_t nip = (size_t)round_up(ni, 64);
     auto a256 = [](size_t b) { return (b + 255) & ~(size_t)255; };
-    const size_t o_nbc = a256(sizeof(ClusterDesc));
+    const size_t o_nbc = 256;
     const size_t o_nbl = o_nbc + a256(nip * sizeof(int));
     const size_t o_part = o_nbl + a256(nip * (size_t)cap * sizeof(int));
     const int ns_min = 1;
     REQUIRE(o_part + nip * ns_min * 8 * sizeof(double) <= kNoAllocBytes,
             "gpunb_regf_dev_noalloc: ni * nnbmax too large for the 48 MiB "
             "scratch (use gpunb_regf_dev)");
-    int ns = ntile == 0 ? 1 : decompose(ni, ntile, m_flag, group, prec);
+    int ju = 6;
+    int ns = ntile == 0 ? 1 : decompose(ni, ntile, m_flag, group, prec, ju);
     const size_t fit = (kNoAllocBytes - o_part) / (nip * 8 * sizeof(double));
     ns = (int)std::max<size_t>(ns_min, std::min<size_t>(ns, fit));
     ClusterDesc D;
@@ -733,11 +721,10 @@ void enqueue_regf_noalloc(int ni, const double *xi, const double *vi,
     D.ni = ni;
     D.n_iw = cdiv(ni, 64);
     D.nslice = ns;
+    D.ju = ju;
     D.cap = cap;
     D.ipb = pass2_ipb(ni);
-    ClusterDesc *d_desc = (ClusterDesc *)base;
     int *nbc = (int *)(base + o_nbc);
-    launch_set_desc(S.st, d_desc, D);
     launch_zero_int(S.st, nbc, (int)nip);
     RegfLaunch L;
     memset(&L, 0, sizeof L);
@@ -765,7 +752,7 @@ void enqueue_regf_noalloc(int ni, const double *xi, const double *vi,
     L.group = group;
     L.prec = prec;
     L.err = S.err.p;
-    L.desc = d_desc;
+    L.one = D;
     L.ncl = 1;
     L.ntask = (long long)D.n_iw * D.nslice;
     L.nblk2 = cdiv(D.ni, D.ipb);
@@ -836,7 +823,7 @@ void do_close() {
     }
     set_device();
     HIPCHK(hipStreamSynchronize(S.st));
-    S.ev_send_live = S.ev_jp_live = S.ev_desc_live = false;
+    S.ev_send_live = S.ev_jp_live = false;
     S.jp.release();
     S.sv.release();
     S.d_send.release();
@@ -1428,8 +1415,9 @@ void ens_regf_dev(int ncl, const int *ni, const double *h2, const double *dtr,
         D.n_iw = cdiv(ni[c], 64);
         D.nslice = std::max(1, cdiv(ntile, Lc));
         D.nslice = std::min(D.nslice, std::max(ntile, 1));
+        D.ju = 6;
         D.cap = std::max(nnbmax, 1);
-        D.ipb = pass2_ipb(ni[c]);
+        D.ipb = pass2_ipb((int)ni_all);
         D.jc = c;
         D.ibase = (int)i0;
         D.pbase = pairs;

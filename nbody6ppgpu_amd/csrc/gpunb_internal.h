@@ -155,6 +155,8 @@ struct ClusterDesc {
     int ni;
     int n_iw;          // i wavefronts: ceil(ni / 64)
     int nslice;        // j slices per i wavefront
+    int ju;            // slices are cut in units of 2^ju j (6; the FP64
+                       // kernel also takes 4)
     int cap;           // list entries stored per i (max(nnbmax, 1))
     int ipb;           // pass-2 i per workgroup
     int jc;            // index of the cluster's JClus
@@ -194,8 +196,9 @@ struct RegfLaunch {
     int group;       // pairs per branch-free group of pass 1 (2 or 4)
     int prec;        // 32: FP32 pair arithmetic; 64/65: FP64 (+ Newton steps)
     unsigned *err;
-    // cluster table (device) and grid sizes
+    // clusters: a device table (ensemble), or NULL and one by value
     const ClusterDesc *desc;
+    ClusterDesc one;
     int ncl;
     long long ntask;   // pass-1 tasks over all clusters
     long long nblk2;   // pass-2 workgroups over all clusters
@@ -269,15 +272,13 @@ void launch_park_view(hipStream_t st, JRec32 *j32, int n, JTile *tiles,
                       int ntile);
 void launch_regf_pass1(hipStream_t st, const RegfLaunch &L);
 void launch_regf_pass2(hipStream_t st, const RegfLaunch &L);
-int pass2_ipb(int ni);   // pass-2 i per workgroup for a cluster of ni
+int pass2_ipb(int ni);   // pass-2 i per workgroup for a launch of ni
 // Entries of a pass-2 wavefront's LDS list row (>= nnbmax + 1); the row of
 // the four wavefronts of a workgroup must fit the 64 KiB of LDS a
 // workgroup can address, hence the largest supported nnbmax.
 int pass2_sortcap(int nnbmax);
 constexpr int kMaxNnbmax = 4000;
 void launch_zero_int(hipStream_t st, int *p, int n);
-// *d = v, in stream order (a cluster table without a host buffer).
-void launch_set_desc(hipStream_t st, ClusterDesc *d, const ClusterDesc &v);
 // bytes (a multiple of 16, both pointers 16-byte aligned) from device memory
 // to a mapped pinned host buffer, and *err to *herr (host-mapped).
 void launch_copy_to_host(hipStream_t st, const void *src, void *dst,

@@ -24,6 +24,7 @@
 #include <cfloat>
 #include <climits>
 #include <cmath>
+#include <type_traits>
 
 namespace gpunb {
 
@@ -302,24 +303,65 @@ __global__ __launch_bounds__(256) void k_copy_from_host(
     if (blockIdx.x == 0 && threadIdx.x == 0) *zero = 0;
 }
 
-__global__ void k_set_desc(ClusterDesc *d, ClusterDesc v) { *d = v; }
-
 __global__ void k_zero_int(int *p, int n) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k < n) p[k] = 0;
 }
+
+// LDS of a pass-1 workgroup, one part per wavefront: while the pair loops
+// run it holds the list entries found (row k: entry k of every lane), after
+// them the wavefront's FP64 sums.  Both are kHitRows * 64 ints.
+constexpr int kHitRows = 14;
+static_assert(kHitRows * 64 * sizeof(int) == 7 * 64 * sizeof(double),
+              "the list entries and the sums share a wavefront's LDS");
+struct alignas(16) P1Lds {
+    int w[kP1W][kHitRows * 64];
+};
+
+// The list entries of one lane (i).  They are kept in LDS and appended to
+// the i's row of nbl a batch at a time, with one returning atomic per batch.
+// An atomic per entry costs the wavefront a memory round trip inside the
+// pair loop, which is all of a small call: N = 1000, 20 i, pass 1 34.5 us
+// with one atomic per entry and a tile per wavefront, 9.9 us so and with 16
+// j per wavefront.
+struct HitList {
+    int *lds;     // the lane's column of its wavefront's rows
+    int n;
+    int i;
+    int *nbc;     // counts and entries of the cluster's i
+    int *nbl;
+    int cap;
+    __device__ __forceinline__ void flush() {
+        if (n > 0) {
+            // Slices append in any order (pass 2 sorts); entries beyond cap
+            // only count (overflow).
+            const int base = atomicAdd(&nbc[i], n);
+            int *row = nbl + (size_t)i * cap + base;
+            for (int k = 0; k < n; ++k)
+                if (base + k < cap) row[k] = lds[64 * k];
+            n = 0;
+        }
+    }
+    __device__ __forceinline__ void push(int j) {
+        lds[64 * n] = j;
+        if (++n == kHitRows) flush();
+    }
+};
 
 // The kP1W wavefronts of a pass-1 workgroup share one (i-wavefront, j
 // slice) task, each over a contiguous part of the slice's tiles; their FP64
 // sums are added in wavefront order through LDS and the first wavefront
 // writes the slice partial of its lanes (a fixed order: the results do not
 // depend on which wavefront finishes first).
-__device__ inline void slice_partial_store(const double (&v)[7], int wv,
-                                           int lane, bool act, double *p) {
-    __shared__ double red[kP1W - 1][7][64];
+__device__ inline void slice_partial_store(P1Lds &lds, const double (&v)[7],
+                                           int wv, int lane, bool act,
+                                           double *p) {
+    // A wavefront's sums replace its own list entries, already appended.
+    asm volatile("" ::: "memory");
+    double *red = reinterpret_cast<double *>(lds.w[wv]);
     if (wv > 0) {
 #pragma unroll
-        for (int c = 0; c < 7; ++c) red[wv - 1][c][lane] = v[c];
+        for (int c = 0; c < 7; ++c) red[64 * c + lane] = v[c];
     }
     __syncthreads();
     if (wv == 0 && act) {
@@ -327,7 +369,8 @@ __device__ inline void slice_partial_store(const double (&v)[7], int wv,
         for (int c = 0; c < 7; ++c) {
             double t = v[c];
 #pragma unroll
-            for (int w = 0; w < kP1W - 1; ++w) t += red[w][c][lane];
+            for (int w = 1; w < kP1W; ++w)
+                t += reinterpret_cast<const double *>(lds.w[w])[64 * c + lane];
             p[c] = t;
         }
         p[7] = 0.0;
@@ -378,7 +421,10 @@ __device__ inline double f64_screen_thr(double h2d, double dtrd, double u0,
 // Near tiles: the FP64 pair loop of k_regf_pass1_f64 (FP64 differences of
 // the sorted FP64 records, 1/r by v_rsq_f64 and one Newton step, the
 // oracle's neighbour predicate bit for bit on the pairs its screen cannot
-// decide), accumulating into the FP64 sums directly.
+// decide), accumulating into the FP64 sums directly.  The band reaches
+// sqrt(K) = 3.5 neighbour radii, so most near tiles hold no neighbour of any
+// lane; where the bounds below show that, the loop runs without the screen
+// (32 instead of 37 FP64 instructions a pair).
 //
 // The split.  FP32 rounding of a pair term is harmless unless the pair is
 // close: relative to the neighbour sphere, and more so for heavy j whose
@@ -416,6 +462,14 @@ __device__ inline void opaque_sgpr(JRec &r) {
                       "+s"(r.vy), "+s"(r.vz), "+s"(r.m));
 }
 
+// Opaque copy of a VGPR value: what is computed from it is computed again
+// (the rare exact predicate forms its differences from it, instead of the
+// pair loop holding twelve registers a pair for its sake).
+__device__ inline double again(double v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
 // Task of a cluster -> (j slice s, i wavefront iw).  XCD x runs the x-th
 // eighth of a launch's tasks (xcd_task).  Slice-major order gives it a share
 // of the slices over most of the i.  In a one-cluster launch of at least
@@ -446,15 +500,13 @@ __device__ __forceinline__ void regf_pass1_task(
     long long gtask,
     const JRec32 *__restrict__ j32_all, const JTile *__restrict__ tile_all,
     const JRec *__restrict__ jps_all, const JClus *__restrict__ jcl_all,
-    const ClusterDesc *__restrict__ desc, int ncl, long long ntask,
-    const JStats *__restrict__ jst, const double *__restrict__ xi_all,
+    const ClusterDesc &D, int ncl, const JStats *__restrict__ jst, const double *__restrict__ xi_all,
     const double *__restrict__ vi_all, const double *__restrict__ h2_all,
     const double *__restrict__ dtr_all, double *__restrict__ part_all,
     int *__restrict__ nbc_all, int *__restrict__ nbl_all,
-    unsigned *__restrict__ err) {
-    const ClusterDesc &D = desc[find_task(desc, ncl, gtask)];
+    unsigned *__restrict__ err, P1Lds &lds) {
     const int nj = D.nj, ntile = D.ntile, ni = D.ni, n_iw = D.n_iw;
-    const int nslice = D.nslice, cap = D.cap;
+    const int nslice = D.nslice;
     const JRec32 *__restrict__ j32 = j32_all + D.j0;
     const JTile *__restrict__ tiles = tile_all + D.j0 / kVTile;
     const JRec *__restrict__ jps = jps_all + D.j0;
@@ -464,8 +516,6 @@ __device__ __forceinline__ void regf_pass1_task(
     const double *__restrict__ h2 = h2_all + D.i0;
     const double *__restrict__ dtr = dtr_all + D.i0;
     double *__restrict__ part = part_all + 8 * D.pbase;
-    int *__restrict__ nbc = nbc_all + D.ibase;
-    int *__restrict__ nbl = nbl_all + D.sbase;
     const int task = (int)(gtask - D.task0);
     int s, iw;
     task_slice(task, n_iw, nslice, ncl == 1, s, iw);
@@ -475,6 +525,8 @@ __device__ __forceinline__ void regf_pass1_task(
     const int lane = threadIdx.x & 63;
     const int i = iw * 64 + lane;
     const bool act = i < ni;
+    HitList hit = {lds.w[wv] + lane, 0, i, nbc_all + D.ibase,
+                   nbl_all + D.sbase, D.cap};
 
     // Slice s of the j tiles, and this wavefront's contiguous share of it.
     const int sb = (int)(((long long)ntile * s) / nslice);
@@ -483,10 +535,11 @@ __device__ __forceinline__ void regf_pass1_task(
     const int te = sb + (int)(((long long)(se - sb) * (wv + 1)) / kP1W);
 
     double x0 = 0.0, y0 = 0.0, z0 = 0.0, u0 = 0.0, w0 = 0.0, q0 = 0.0;
-    double h2d = 0.0, dtrd = 0.0, dtr2x = 0.0;   // dtr2x = 2 dtr
+    double dtr2x = 0.0;         // 2 dtr
     double thr = -1.0;          // FP64 screen threshold (k_regf_pass1_f64)
     float adtr = 0.0f;          // >= |dtr|
     float B = 0.0f;             // band base
+    float hrad = 0.0f;          // >= sqrt(h2) (sqrt(h2 <m>) mass-weighted)
     if (act) {
         x0 = xi[3 * (size_t)i + 0];
         y0 = xi[3 * (size_t)i + 1];
@@ -494,8 +547,7 @@ __device__ __forceinline__ void regf_pass1_task(
         u0 = vi[3 * (size_t)i + 0];
         w0 = vi[3 * (size_t)i + 1];
         q0 = vi[3 * (size_t)i + 2];
-        h2d = h2[i];
-        dtrd = dtr[i];
+        const double h2d = h2[i], dtrd = dtr[i];
         dtr2x = 2.0 * dtrd;
         const double chk = x0 + y0 + z0 + u0 + w0 + q0 + h2d + dtrd;
         if (chk != chk) atomicOr(err, ERR_NAN_I);
@@ -504,6 +556,7 @@ __device__ __forceinline__ void regf_pass1_task(
             const double bb = (double)kBand * h2d * (MFLAG ? mbar : 1.0) *
                               (1.0 + 8.0 * (double)kU32);
             B = (float)bb * (1.0f + 2.0f * kU32);
+            hrad = sqrtf(B / kBand) * (1.0f + 1e-5f);
             thr = f64_screen_thr<MFLAG>(h2d, dtrd, u0, w0, q0, jst);
         } else {
             thr = 1e-30;
@@ -515,20 +568,20 @@ __device__ __forceinline__ void regf_pass1_task(
     // FP64 pair of a near tile: the screen of k_regf_pass1_f64, the exact
     // predicate for the pairs it flags.
     auto resolve = [&](const JRec &J, int j) {
-        const double dx = J.x - x0, dy = J.y - y0, dz = J.z - z0;
-        const double dvx = J.vx - u0, dvy = J.vy - w0, dvz = J.vz - q0;
+        const double dx = J.x - again(x0), dy = J.y - again(y0),
+                     dz = J.z - again(z0);
+        const double dvx = J.vx - again(u0), dvy = J.vy - again(w0),
+                     dvz = J.vz - again(q0);
         const double r2d = sq3d(dx, dy, dz);
+        const double dtrd = 0.5 * dtr2x;   // exact
         const double pxd = dx + dtrd * dvx;
         const double pyd = dy + dtrd * dvy;
         const double pzd = dz + dtrd * dvz;
         const double r2pd = sq3d(pxd, pyd, pzd);
         const double mnd = r2d < r2pd ? r2d : r2pd;
-        const double H = MFLAG ? J.m * h2d : h2d;
+        const double H = MFLAG ? J.m * h2[i] : h2[i];
         if ((mnd < H) && (j < nj)) {
-            // Slices append in any order (pass 2 sorts); entries beyond cap
-            // only count (overflow).
-            const int k2 = atomicAdd(&nbc[i], 1);
-            if (k2 < cap) nbl[(size_t)i * cap + k2] = j;
+            hit.push(j);
         } else if (r2d != 0.0) {
             // Rare (band pairs, r2 < 1e-30): exact FP64 1/sqrt.
             const double rinv = 1.0 / sqrt(r2d);
@@ -565,13 +618,17 @@ __device__ __forceinline__ void regf_pass1_task(
         const float Vx = (float)(T.cu - u0), Vy = (float)(T.cv - w0),
                     Vz = (float)(T.cw - q0);
         const float Bt = fmaxf(B, T.eb);
-        const float d = sqrtf(fmaf(Dz, Dz, fmaf(Dy, Dy, Dx * Dx)));
-        const float dvn = sqrtf(fmaf(Vz, Vz, fmaf(Vy, Vy, Vx * Vx)));
+        // v_sqrt_f32 (1 ulp): far inside the margins.
+        const float d =
+            __builtin_amdgcn_sqrtf(fmaf(Dz, Dz, fmaf(Dy, Dy, Dx * Dx)));
+        const float dvn =
+            __builtin_amdgcn_sqrtf(fmaf(Vz, Vz, fmaf(Vy, Vy, Vx * Vx)));
         const float R = fmaf(d, 1.0f - 1e-5f, -T.e);
         const float A = adtr * (dvn + T.ev) * (1.0f + 1e-5f);
         const float Tmax = Bt * T.wmax * (1.0f + 1e-5f);
         const bool far =
-            !act || (R > fmaf(sqrtf(fmaf(A, A, Tmax)), 1.0f + 1e-5f, A));
+            !act || (R > fmaf(__builtin_amdgcn_sqrtf(fmaf(A, A, Tmax)),
+                              1.0f + 1e-5f, A));
         if (__ballot(!far) == 0) {
             float ax = 0.f, ay = 0.f, az = 0.f, jx = 0.f, jy = 0.f, jz = 0.f,
                   ph = 0.f;
@@ -619,9 +676,10 @@ __device__ __forceinline__ void regf_pass1_task(
             Jz += (double)jz;
             Ph += (double)ph;
         } else {
-            // FP64 group of G records at sorted position jb: the screen
-            // flags the pairs the exact predicate decides.
-            auto group64 = [&](const JRec (&J)[G], int jb) {
+            // FP64 group of G records at sorted position jb.  SCREEN: the
+            // screen flags the pairs the exact predicate decides.
+            auto group64 = [&](const JRec (&J)[G], int jb, auto screen) {
+                constexpr bool SCREEN = decltype(screen)::value;
                 bool fl[G];
                 bool any = false;
 #pragma unroll
@@ -634,16 +692,18 @@ __device__ __forceinline__ void regf_pass1_task(
                     const double dvz = J[k].vz - q0;
                     const double r2 = fma(dz, dz, fma(dy, dy, dx * dx));
                     const double rv = fma(dz, dvz, fma(dy, dvy, dx * dvx));
-                    const double q = fma(dtr2x, rv, r2);
-                    double tj = thr;
-                    if (MFLAG) tj = fmax(thr * J[k].m, 1e-30);
-                    fl[k] = fmin(r2, q) < tj;
-                    any = any || fl[k];
                     double y = __builtin_amdgcn_rsq(r2);
                     y = fma(y, 0.5 * fma(-r2 * y, y, 1.0), y);
-                    const double rinv = fl[k] ? 0.0 : y;
-                    const double rinv2 = rinv * rinv;
-                    const double mr = J[k].m * rinv;
+                    if constexpr (SCREEN) {
+                        const double q = fma(dtr2x, rv, r2);
+                        double tj = thr;
+                        if (MFLAG) tj = fmax(thr * J[k].m, 1e-30);
+                        fl[k] = fmin(r2, q) < tj;
+                        any = any || fl[k];
+                        y = fl[k] ? 0.0 : y;
+                    }
+                    const double rinv2 = y * y;
+                    const double mr = J[k].m * y;
                     const double mr3 = mr * rinv2;
                     const double al = (-3.0 * rv) * rinv2;
                     Ph += mr;
@@ -654,31 +714,51 @@ __device__ __forceinline__ void regf_pass1_task(
                     Jy = fma(mr3, fma(al, dy, dvy), Jy);
                     Jz = fma(mr3, fma(al, dz, dvz), Jz);
                 }
-                if (any) {
+                if constexpr (SCREEN) {
+                    if (any) {
 #pragma unroll
-                    for (int k = 0; k < G; ++k)
-                        if (fl[k]) resolve(J[k], jb + k);
+                        for (int k = 0; k < G; ++k)
+                            if (fl[k]) resolve(J[k], jb + k);
+                    }
                 }
             };
-            JRec Pa[G], Pb[G];
+            auto tile64 = [&](auto screen) {
+                JRec Pa[G], Pb[G];
 #pragma unroll
-            for (int k = 0; k < G; ++k) {
-                Pa[k] = jps[jt + k];
-                opaque_sgpr(Pa[k]);
-            }
-            for (int jg = 0; jg < kVTile; jg += 2 * G) {
+                for (int k = 0; k < G; ++k) {
+                    Pa[k] = jps[jt + k];
+                    opaque_sgpr(Pa[k]);
+                }
+                for (int jg = 0; jg < kVTile; jg += 2 * G) {
 #pragma unroll
-                for (int k = 0; k < G; ++k) Pb[k] = jps[jt + jg + G + k];
-                group64(Pa, jt + jg);
+                    for (int k = 0; k < G; ++k) Pb[k] = jps[jt + jg + G + k];
+                    group64(Pa, jt + jg, screen);
 #pragma unroll
-                for (int k = 0; k < G; ++k) Pa[k] = jps[jt + jg + 2 * G + k];
-                group64(Pb, jt + jg + G);
-            }
+                    for (int k = 0; k < G; ++k)
+                        Pa[k] = jps[jt + jg + 2 * G + k];
+                    group64(Pb, jt + jg + G, screen);
+                }
+            };
+            // (R - A)^2 > H for every pair: no neighbour in the tile.  With
+            // mass-weighted lists H = m_j h2 and x_j = m_j / <m> follows
+            // from w_j >= max(x^(2/3), 1.4 x / K): x <= min(w^(3/2), K w /
+            // 1.4).
+            float hr = hrad;
+            if (MFLAG)
+                hr *= __builtin_amdgcn_sqrtf(
+                    fminf(T.wmax * __builtin_amdgcn_sqrtf(T.wmax),
+                          kBand / 1.4f * T.wmax)) * (1.0f + 1e-5f);
+            const bool none = !act || R > A + hr;
+            if (__ballot(!none) == 0)
+                tile64(std::false_type());
+            else
+                tile64(std::true_type());
         }
     }
 
+    hit.flush();
     double sums[7] = {Ax, Ay, Az, Jx, Jy, Jz, Ph};
-    slice_partial_store(sums, wv, lane, act,
+    slice_partial_store(lds, sums, wv, lane, act,
                         part + ((size_t)s * n_iw * 64 + i) * 8);
 }
 
@@ -702,23 +782,19 @@ __device__ __forceinline__ void regf_pass1_task(
 template <bool MFLAG, int G, int NR>
 __device__ __forceinline__ void regf_pass1_f64_task(
     long long gtask,
-    const JRec *__restrict__ jp_all, const ClusterDesc *__restrict__ desc,
-    int ncl, long long ntask, const JStats *__restrict__ jst,
+    const JRec *__restrict__ jp_all, const ClusterDesc &D, int ncl, const JStats *__restrict__ jst,
     const double *__restrict__ xi_all, const double *__restrict__ vi_all,
     const double *__restrict__ h2_all, const double *__restrict__ dtr_all,
     double *__restrict__ part_all, int *__restrict__ nbc_all,
-    int *__restrict__ nbl_all, unsigned *__restrict__ err) {
-    const ClusterDesc &D = desc[find_task(desc, ncl, gtask)];
+    int *__restrict__ nbl_all, unsigned *__restrict__ err, P1Lds &lds) {
     const int nj = D.nj, ntile = D.ntile, ni = D.ni, n_iw = D.n_iw;
-    const int nslice = D.nslice, cap = D.cap;
+    const int nslice = D.nslice;
     const JRec *__restrict__ jp = jp_all + D.j0;
     const double *__restrict__ xi = xi_all + 3 * (size_t)D.i0;
     const double *__restrict__ vi = vi_all + 3 * (size_t)D.i0;
     const double *__restrict__ h2 = h2_all + D.i0;
     const double *__restrict__ dtr = dtr_all + D.i0;
     double *__restrict__ part = part_all + 8 * D.pbase;
-    int *__restrict__ nbc = nbc_all + D.ibase;
-    int *__restrict__ nbl = nbl_all + D.sbase;
     const int task = (int)(gtask - D.task0);
     int s, iw;
     task_slice(task, n_iw, nslice, ncl == 1, s, iw);
@@ -728,15 +804,21 @@ __device__ __forceinline__ void regf_pass1_f64_task(
     const int lane = threadIdx.x & 63;
     const int i = iw * 64 + lane;
     const bool act = i < ni;
+    HitList hit = {lds.w[wv] + lane, 0, i, nbc_all + D.ibase,
+                   nbl_all + D.sbase, D.cap};
 
-    // Slice s of the j tiles, and this wavefront's contiguous share of it.
-    const int sb = (int)(((long long)ntile * s) / nslice);
-    const int se = (int)(((long long)ntile * (s + 1)) / nslice);
-    const int tb = sb + (int)(((long long)(se - sb) * wv) / kP1W);
-    const int te = sb + (int)(((long long)(se - sb) * (wv + 1)) / kP1W);
+    // Slice s of the j (in units of 2^ju of them), and this wavefront's
+    // contiguous share of it.
+    const int nu = ntile << (6 - D.ju);
+    const int sb = (int)(((long long)nu * s) / nslice);
+    const int se = (int)(((long long)nu * (s + 1)) / nslice);
+    const int jb = __builtin_amdgcn_readfirstlane(
+        (sb + (int)(((long long)(se - sb) * wv) / kP1W)) << D.ju);
+    const int je = __builtin_amdgcn_readfirstlane(
+        (sb + (int)(((long long)(se - sb) * (wv + 1)) / kP1W)) << D.ju);
 
     double x0 = 0.0, y0 = 0.0, z0 = 0.0, u0 = 0.0, w0 = 0.0, q0 = 0.0;
-    double h2d = 0.0, dtrd = 0.0, dtr2x = 0.0;   // dtr2x = 2 dtr
+    double dtr2x = 0.0;   // 2 dtr
     double thr = -1.0;
     if (act) {
         x0 = xi[3 * (size_t)i + 0];
@@ -745,8 +827,7 @@ __device__ __forceinline__ void regf_pass1_f64_task(
         u0 = vi[3 * (size_t)i + 0];
         w0 = vi[3 * (size_t)i + 1];
         q0 = vi[3 * (size_t)i + 2];
-        h2d = h2[i];
-        dtrd = dtr[i];
+        const double h2d = h2[i], dtrd = dtr[i];
         dtr2x = 2.0 * dtrd;
         const double chk = x0 + y0 + z0 + u0 + w0 + q0 + h2d + dtrd;
         if (chk != chk) atomicOr(err, ERR_NAN_I);
@@ -793,18 +874,20 @@ __device__ __forceinline__ void regf_pass1_f64_task(
     };
 
     auto resolve = [&](const JRec &J, int j) {
-        const double dx = J.x - x0, dy = J.y - y0, dz = J.z - z0;
-        const double dvx = J.vx - u0, dvy = J.vy - w0, dvz = J.vz - q0;
+        const double dx = J.x - again(x0), dy = J.y - again(y0),
+                     dz = J.z - again(z0);
+        const double dvx = J.vx - again(u0), dvy = J.vy - again(w0),
+                     dvz = J.vz - again(q0);
         const double r2d = sq3d(dx, dy, dz);
+        const double dtrd = 0.5 * dtr2x;   // exact
         const double pxd = dx + dtrd * dvx;
         const double pyd = dy + dtrd * dvy;
         const double pzd = dz + dtrd * dvz;
         const double r2pd = sq3d(pxd, pyd, pzd);
         const double mnd = r2d < r2pd ? r2d : r2pd;
-        const double H = MFLAG ? J.m * h2d : h2d;
+        const double H = MFLAG ? J.m * h2[i] : h2[i];
         if ((mnd < H) && (j < nj)) {
-            const int k2 = atomicAdd(&nbc[i], 1);
-            if (k2 < cap) nbl[(size_t)i * cap + k2] = j;
+            hit.push(j);
         } else if (r2d != 0.0) {
             // Rare (band pairs, r2 < 1e-30): exact FP64 1/sqrt.
             const double rv = fma(dz, dvz, fma(dy, dvy, dx * dvx));
@@ -812,55 +895,56 @@ __device__ __forceinline__ void regf_pass1_f64_task(
         }
     };
 
-    // The records of the next group are loaded while the current group is
-    // evaluated, hiding the scalar-load latency inside the wave (5% faster
-    // per launch).  The j array carries 64 spare records past its last tile,
-    // so the look-ahead of the last group stays in bounds.
-    JRec Jn[G];
+    auto group = [&](const JRec (&J)[G], int j0) {
+        bool fl[G];
+        bool any = false;
+#pragma unroll
+        for (int k = 0; k < G; ++k) {
+            const double dx = J[k].x - x0;
+            const double dy = J[k].y - y0;
+            const double dz = J[k].z - z0;
+            const double dvx = J[k].vx - u0;
+            const double dvy = J[k].vy - w0;
+            const double dvz = J[k].vz - q0;
+            const double r2 = fma(dz, dz, fma(dy, dy, dx * dx));
+            const double rv = fma(dz, dvz, fma(dy, dvy, dx * dvx));
+            const double q = fma(dtr2x, rv, r2);
+            double tj = thr;
+            if (MFLAG) tj = fmax(thr * J[k].m, 1e-30);
+            fl[k] = fmin(r2, q) < tj;
+            any = any || fl[k];
+            const double rinv = fl[k] ? 0.0 : rsq64(r2);
+            pair_terms(J[k], dx, dy, dz, dvx, dvy, dvz, rv, rinv);
+        }
+        if (any) {
+#pragma unroll
+            for (int k = 0; k < G; ++k)
+                if (fl[k]) resolve(J[k], j0 + k);
+        }
+    };
+    // Two record buffers in turn: the next group's records load while the
+    // current group is evaluated.  A unit is a whole number of both buffers,
+    // and the j array carries 64 spare records past its last tile, so the
+    // look-ahead of the last group stays in bounds.
+    JRec Pa[G], Pb[G];
 #pragma unroll
     for (int k = 0; k < G; ++k) {
-        Jn[k] = jp[tb * kTile + k];
-        opaque_sgpr(Jn[k]);
+        Pa[k] = jp[jb + k];
+        opaque_sgpr(Pa[k]);
     }
-    for (int t = tb; t < te; ++t) {
-        const int jt = t * kTile;
-        for (int jg = 0; jg < kTile; jg += G) {
-            JRec J[G];
-            bool fl[G];
-            bool any = false;
+    for (int j = jb; j < je; j += 2 * G) {
 #pragma unroll
-            for (int k = 0; k < G; ++k) J[k] = Jn[k];
+        for (int k = 0; k < G; ++k) Pb[k] = jp[j + G + k];
+        group(Pa, j);
 #pragma unroll
-            for (int k = 0; k < G; ++k) Jn[k] = jp[jt + jg + G + k];
-#pragma unroll
-            for (int k = 0; k < G; ++k) {
-                const double dx = J[k].x - x0;
-                const double dy = J[k].y - y0;
-                const double dz = J[k].z - z0;
-                const double dvx = J[k].vx - u0;
-                const double dvy = J[k].vy - w0;
-                const double dvz = J[k].vz - q0;
-                const double r2 = fma(dz, dz, fma(dy, dy, dx * dx));
-                const double rv = fma(dz, dvz, fma(dy, dvy, dx * dvx));
-                const double q = fma(dtr2x, rv, r2);
-                double tj = thr;
-                if (MFLAG) tj = fmax(thr * J[k].m, 1e-30);
-                fl[k] = fmin(r2, q) < tj;
-                any = any || fl[k];
-                const double rinv = fl[k] ? 0.0 : rsq64(r2);
-                pair_terms(J[k], dx, dy, dz, dvx, dvy, dvz, rv, rinv);
-            }
-            if (any) {
-#pragma unroll
-                for (int k = 0; k < G; ++k)
-                    if (fl[k]) resolve(J[k], jt + jg + k);
-            }
-        }
+        for (int k = 0; k < G; ++k) Pa[k] = jp[j + 2 * G + k];
+        group(Pb, j + G);
     }
 
+    hit.flush();
     double sums[7] = {ax, ay, az, fma(-3.0, j2x, j1x), fma(-3.0, j2y, j1y),
                       fma(-3.0, j2z, j1z), ph};
-    slice_partial_store(sums, wv, lane, act,
+    slice_partial_store(lds, sums, wv, lane, act,
                         part + ((size_t)s * n_iw * 64 + i) * 8);
 }
 
@@ -873,6 +957,12 @@ __device__ inline long long xcd_task(long long ntask) {
     const long long t = (long long)(blockIdx.x & 7) * per + (blockIdx.x >> 3);
     return t < ntask ? t : -1;
 }
+
+// Wavefronts per SIMD that the pass-1 kernels are held to (VGPRs).  At G = 2
+// five fit without spills (the FP64 kernel fits six by itself): King N =
+// 131072, whole step, 14.55 ms at four, 14.3 at five, 14.8 at six (15 VGPRs
+// spilled).  At G = 4 the pair groups need the registers of three.
+constexpr int p1_waves(int g) { return g == 2 ? 5 : 3; }
 
 // Next task of a persistent workgroup.  Tasks [xr[x], xr[x + 1]) belong to
 // XCD x (the workgroup's XCD is blockIdx.x & 7: workgroups of a grid that
@@ -903,98 +993,172 @@ __device__ inline long long next_task(unsigned *__restrict__ q,
         s_task = t;
     }
     __syncthreads();
-    return s_task;
+    // Uniform in SGPRs: what depends on the task (the j record addresses)
+    // stays scalar.
+    const long long t = s_task;
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)t);
+    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(t >> 32));
+    return (long long)(((unsigned long long)hi << 32) | lo);
 }
 
 template <bool MFLAG, int G>
-__global__ __launch_bounds__(64 * kP1W) void k_regf_pass1(
+__global__ __launch_bounds__(64 * kP1W, p1_waves(G)) void k_regf_pass1(
     const JRec32 *__restrict__ j32_all, const JTile *__restrict__ tile_all,
     const JRec *__restrict__ jps_all, const JClus *__restrict__ jcl_all,
-    const ClusterDesc *__restrict__ desc, int ncl, long long ntask,
-    const JStats *__restrict__ jst, const double *__restrict__ xi_all,
+    const ClusterDesc *__restrict__ desc, ClusterDesc one, int ncl,
+    long long ntask, const JStats *__restrict__ jst, const double *__restrict__ xi_all,
     const double *__restrict__ vi_all, const double *__restrict__ h2_all,
     const double *__restrict__ dtr_all, double *__restrict__ part_all,
     int *__restrict__ nbc_all, int *__restrict__ nbl_all,
     unsigned *__restrict__ err) {
+    __shared__ P1Lds lds;
     const long long t = xcd_task(ntask);
     if (t < 0) return;
-    regf_pass1_task<MFLAG, G>(t, j32_all, tile_all, jps_all, jcl_all, desc, ncl, ntask, jst, xi_all, vi_all,
-        h2_all, dtr_all, part_all, nbc_all, nbl_all, err);
+    ClusterDesc D = one;
+    if (desc) D = desc[find_task(desc, ncl, t)];
+    regf_pass1_task<MFLAG, G>(t, j32_all, tile_all, jps_all, jcl_all,
+        D, ncl, jst, xi_all, vi_all, h2_all, dtr_all, part_all,
+        nbc_all, nbl_all, err, lds);
 }
 
 // Persistent form: a grid of resident workgroups takes tasks from the XCD
 // queues until all are done (the ensemble's uneven tasks, largest first).
 template <bool MFLAG, int G>
-__global__ __launch_bounds__(64 * kP1W) void k_regf_pass1_q(
+__global__ __launch_bounds__(64 * kP1W, p1_waves(G)) void k_regf_pass1_q(
     const JRec32 *__restrict__ j32_all, const JTile *__restrict__ tile_all,
     const JRec *__restrict__ jps_all, const JClus *__restrict__ jcl_all,
-    const ClusterDesc *__restrict__ desc, int ncl, long long ntask,
-    const JStats *__restrict__ jst, const double *__restrict__ xi_all,
+    const ClusterDesc *__restrict__ desc, int ncl,
+    long long ntask, const JStats *__restrict__ jst, const double *__restrict__ xi_all,
     const double *__restrict__ vi_all, const double *__restrict__ h2_all,
     const double *__restrict__ dtr_all, double *__restrict__ part_all,
     int *__restrict__ nbc_all, int *__restrict__ nbl_all,
     unsigned *__restrict__ err, unsigned *__restrict__ q, const long long *__restrict__ xr) {
+    __shared__ P1Lds lds;
     int x = blockIdx.x & 7, tries = 0;
     for (;;) {
         const long long t = next_task(q, xr, x, tries);
         if (t < 0) return;
-        regf_pass1_task<MFLAG, G>(t, j32_all, tile_all, jps_all, jcl_all, desc, ncl, ntask, jst, xi_all, vi_all,
-        h2_all, dtr_all, part_all, nbc_all, nbl_all, err);
+        const ClusterDesc &D = desc[find_task(desc, ncl, t)];
+        regf_pass1_task<MFLAG, G>(t, j32_all, tile_all, jps_all, jcl_all,
+        D, ncl, jst, xi_all, vi_all, h2_all, dtr_all, part_all,
+        nbc_all, nbl_all, err, lds);
     }
 }
 
 template <bool MFLAG, int G, int NR>
-__global__ __launch_bounds__(64 * kP1W) void k_regf_pass1_f64(
+__global__ __launch_bounds__(64 * kP1W, p1_waves(G)) void k_regf_pass1_f64(
     const JRec *__restrict__ jp_all, const ClusterDesc *__restrict__ desc,
-    int ncl, long long ntask, const JStats *__restrict__ jst,
+    ClusterDesc one, int ncl, long long ntask, const JStats *__restrict__ jst,
     const double *__restrict__ xi_all, const double *__restrict__ vi_all,
     const double *__restrict__ h2_all, const double *__restrict__ dtr_all,
     double *__restrict__ part_all, int *__restrict__ nbc_all,
     int *__restrict__ nbl_all, unsigned *__restrict__ err) {
+    __shared__ P1Lds lds;
     const long long t = xcd_task(ntask);
     if (t < 0) return;
-    regf_pass1_f64_task<MFLAG, G, NR>(t, jp_all, desc, ncl, ntask, jst, xi_all, vi_all, h2_all, dtr_all,
-        part_all, nbc_all, nbl_all, err);
+    ClusterDesc D = one;
+    if (desc) D = desc[find_task(desc, ncl, t)];
+    regf_pass1_f64_task<MFLAG, G, NR>(t, jp_all, D, ncl, jst, xi_all,
+        vi_all, h2_all, dtr_all, part_all, nbc_all, nbl_all, err, lds);
 }
 
 template <bool MFLAG, int G, int NR>
-__global__ __launch_bounds__(64 * kP1W) void k_regf_pass1_f64_q(
+__global__ __launch_bounds__(64 * kP1W, p1_waves(G)) void k_regf_pass1_f64_q(
     const JRec *__restrict__ jp_all, const ClusterDesc *__restrict__ desc,
     int ncl, long long ntask, const JStats *__restrict__ jst,
     const double *__restrict__ xi_all, const double *__restrict__ vi_all,
     const double *__restrict__ h2_all, const double *__restrict__ dtr_all,
     double *__restrict__ part_all, int *__restrict__ nbc_all,
     int *__restrict__ nbl_all, unsigned *__restrict__ err, unsigned *__restrict__ q, const long long *__restrict__ xr) {
+    __shared__ P1Lds lds;
     int x = blockIdx.x & 7, tries = 0;
     for (;;) {
         const long long t = next_task(q, xr, x, tries);
         if (t < 0) return;
-        regf_pass1_f64_task<MFLAG, G, NR>(t, jp_all, desc, ncl, ntask, jst, xi_all, vi_all, h2_all, dtr_all,
-        part_all, nbc_all, nbl_all, err);
+        const ClusterDesc &D = desc[find_task(desc, ncl, t)];
+        regf_pass1_f64_task<MFLAG, G, NR>(t, jp_all, D, ncl, jst, xi_all,
+        vi_all, h2_all, dtr_all, part_all, nbc_all, nbl_all, err, lds);
     }
 }
 
 // ---------------------------------------------------------------------------
 // Regular force, pass 2: a workgroup of 4 wavefronts serves ipb <= kP2I
-// i-particles (ipb chosen per launch so that small calls still spread over
-// the machine), each wavefront every 4th of them.  Per i: the slice partials
-// are summed in a fixed order (deterministic FP64) and the forces written,
-// and the list count read (and reset for the next launch on this scratch);
-// then one thread scans the block's list lengths and claims the block's list
-// space with a single atomic; then every i's list entries (sorted positions,
-// appended by the slices in any order) are mapped to original j indices in
-// the wavefront's LDS row and each written at its rank among them, so the
-// list comes out ascending whatever the append order was; the nearest
-// neighbour (smallest FP64 r2 > 0, ties to the smaller j) is found on the
-// way.
+// consecutive i (ipb chosen per launch so that small calls still spread over
+// the machine), each wavefront a quarter of them.
+//
+// Sums: the lanes of a wavefront are 8 components x P consecutive i x G
+// slice groups (P G = 8): a load takes whole 64-byte partial records, P of
+// them side by side, and only the G groups are added across lanes, in a
+// fixed order (deterministic FP64).
+//
+// Lists: the list entries (sorted positions, appended by the slices in any
+// order) are mapped to the caller's j indices and written in ascending order
+// at the place claimed for them: one atomic per workgroup, on a scan of its
+// list lengths.  The entries of all the wavefront's i are loaded before that
+// and their index gathers run together, so that a wavefront waits for a few
+// memory round trips in all, not for a few per i.  A list of up to 64 is one
+// entry per lane, placed by its rank among the others (16-byte broadcast
+// reads of the LDS row).  A longer one is ranked in chunks of 64 and its
+// entries placed by binary search in the other chunks: n^2 / 64 compares per
+// lane would make the longest lists the launch's end.
+//
+// Bound: latency (a wavefront's chain of dependent loads).  Before, an i at a
+// time with lanes over the slices, every entry ranked against all others:
+// 1024 i of N = 15565 with mass-weighted lists 190 us, now 42 us; 114k i of
+// 24 clusters 360 -> 90 us; 1024 i of N = 131072 16.5 -> 11 us.
+//
+// The nearest neighbour (NN; smallest FP64 r2 > 0, ties to the smaller j) is
+// searched only when the caller asks for it: it costs a record gather per
+// list entry.
+//
+// The list counts are reset for the next launch on this scratch.
 // ---------------------------------------------------------------------------
 
 constexpr int kP2I = 32;
-constexpr int kP2U = 4;   // 64-slice chunks per pass-2 load batch
+constexpr int kP2W = kP2I / 4;   // i per wavefront, at most
+constexpr int kP2U = 8;          // slice partials loaded together
 
+// Entries of the ascending LDS run a[0, m) (m <= 64) below v.
+__device__ inline int run_below(const int *a, int m, int v) {
+    int pos = 0;
+#pragma unroll
+    for (int s = 32; s >= 1; s >>= 1)
+        if (pos + s <= m && a[pos + s - 1] < v) pos += s;
+    return pos + ((pos < m && a[pos] < v) ? 1 : 0);
+}
+
+// Entries below v among the first n of an LDS row (n rounded up to 4 reads
+// padding of INT_MAX), four per read.
+__device__ inline int row_below(const int *row, int n, int v) {
+    const int4 *r4 = reinterpret_cast<const int4 *>(row);
+    int below = 0;
+    for (int k = 0; 4 * k < n; ++k) {
+        const int4 w = r4[k];
+        below += (w.x < v) + (w.y < v) + (w.z < v) + (w.w < v);
+    }
+    return below;
+}
+
+// The lane's (r2, j) minimum over the wavefront, r2 first: the winning j (-1
+// if every r2 is infinite).
+__device__ inline int wave_nearest(double r2, int j) {
+    double m = r2;
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) m = fmin(m, __shfl_xor(m, o));
+    if (!(m < INFINITY)) return -1;
+    unsigned long long at = __ballot(r2 == m);
+    int best = INT_MAX;
+    while (at) {
+        best = min(best, __builtin_amdgcn_readlane(j, __builtin_ctzll(at)));
+        at &= at - 1;
+    }
+    return best;
+}
+
+template <bool NN>
 __global__ __launch_bounds__(256) void k_regf_pass2(
     const JRec *__restrict__ jps_all, const int *__restrict__ jidx_all,
-    const ClusterDesc *__restrict__ desc, int ncl,
+    const ClusterDesc *__restrict__ desc, ClusterDesc one, int ncl,
     const double *__restrict__ xi_all, const double *__restrict__ part_all,
     int *__restrict__ nbc_all, const int *__restrict__ nbl_all,
     double *__restrict__ acc_all, double *__restrict__ jrk_all,
@@ -1005,18 +1169,18 @@ __global__ __launch_bounds__(256) void k_regf_pass2(
     unsigned *__restrict__ err) {
     __shared__ int s_tot[kP2I];
     __shared__ int s_off[kP2I];
-    extern __shared__ int s_rows[];   // [4][sortcap]: one list row per wave
+    extern __shared__ __align__(16) int s_rows[];   // [4][sortcap]
     const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const ClusterDesc &D = desc[find_blk(desc, ncl, blockIdx.x)];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    ClusterDesc D = one;
+    if (desc) D = desc[find_blk(desc, ncl, blockIdx.x)];
     const int ni = D.ni, nslice = D.nslice, cap = D.cap;
-    const int ipb = D.ipb;
-    const int i0 = (int)(blockIdx.x - D.blk0) * ipb;
+    const int ipb = D.ipb, niw = ipb >> 2;
+    const int ib = (int)(blockIdx.x - D.blk0) * ipb + wave * niw;
     const JRec *__restrict__ jps = jps_all + D.j0;
     // NULL: the j records are in the caller's order (position = index).
     const int *__restrict__ jidx = jidx_all ? jidx_all + D.j0 : nullptr;
     const double *__restrict__ xi = xi_all + 3 * (size_t)D.i0;
-    const double *__restrict__ part = part_all + 8 * D.pbase;
     int *__restrict__ nbc = nbc_all + D.ibase;
     const int *__restrict__ nbl = nbl_all + D.sbase;
     // Output row of local i: the caller's index (through perm when the i
@@ -1026,129 +1190,165 @@ __global__ __launch_bounds__(256) void k_regf_pass2(
         return (size_t)(perm ? perm[g] : g);
     };
 
-    for (int r = wave; r < ipb; r += 4) {
-        const int i = i0 + r;
-        int tot = 0;
-        if (i < ni) {
-            // kP2U chunks of 64 slices per batch: their partials are loaded
-            // together, then added in slice order per lane.
-            double sum[7] = {0, 0, 0, 0, 0, 0, 0};
-            for (int b0 = 0; b0 < nslice; b0 += 64 * kP2U) {
-                double v[kP2U][7];
+    // List counts, one i per lane, and the entries of the short lists.
+    int tot = 0;
+    if (lane < niw && ib + lane < ni) tot = nbc[ib + lane];
+    int ent[kP2W], jj[kP2W];
+#pragma unroll
+    for (int r = 0; r < kP2W; ++r) {
+        const int n = __builtin_amdgcn_readlane(tot, r);
+        ent[r] = -1;
+        if (n <= 64 && n <= nnbmax && lane < n)
+            ent[r] = nbl[(size_t)(ib + r) * cap + lane];
+    }
+
+    // Sums.
+    {
+        const int lp = niw >= 8 ? 3 : niw >= 4 ? 2 : niw >= 2 ? 1 : 0;
+        const int P = 1 << lp, G = 8 >> lp;
+        const int c = lane & 7, g = (lane >> 3) >> lp;
+        const size_t stride = (size_t)D.n_iw * 64 * 8;
+        for (int b = 0; b < niw; b += P) {
+            const int i = ib + b + ((lane >> 3) & (P - 1));
+            const bool ok = i < ni;
+            const double *p =
+                part_all + 8 * D.pbase + (size_t)i * 8 + c + g * stride;
+            double sum = 0.0;
+            for (int s0 = g; s0 < nslice; s0 += G * kP2U) {
+                double v[kP2U];
 #pragma unroll
                 for (int u = 0; u < kP2U; ++u) {
-                    const int q = b0 + 64 * u + lane;
-                    if (q < nslice) {
-                        const double *p =
-                            part + ((size_t)q * D.n_iw * 64 + i) * 8;
-#pragma unroll
-                        for (int k = 0; k < 7; ++k) v[u][k] = p[k];
-                    } else {
-#pragma unroll
-                        for (int k = 0; k < 7; ++k) v[u][k] = 0.0;
-                    }
+                    v[u] = ok && s0 + u * G < nslice ? *p : 0.0;
+                    p += G * stride;
                 }
 #pragma unroll
-                for (int u = 0; u < kP2U; ++u) {
-                    if (b0 + 64 * u + lane < nslice) {
-#pragma unroll
-                        for (int k = 0; k < 7; ++k) sum[k] += v[u][k];
-                    }
-                }
+                for (int u = 0; u < kP2U; ++u) sum += v[u];
             }
-#pragma unroll
-            for (int k = 0; k < 7; ++k)
-                for (int o = 32; o >= 1; o >>= 1)
-                    sum[k] += __shfl_xor(sum[k], o);
-            tot = nbc[i];
-            if (lane == 0) {
+            for (int o = 8 * P; o < 64; o <<= 1) sum += __shfl_xor(sum, o);
+            if (ok && g == 0 && c < 7) {
                 const size_t q = orow(i);
-                acc_all[3 * q + 0] = sum[0];
-                acc_all[3 * q + 1] = sum[1];
-                acc_all[3 * q + 2] = sum[2];
-                jrk_all[3 * q + 0] = sum[3];
-                jrk_all[3 * q + 1] = sum[4];
-                jrk_all[3 * q + 2] = sum[5];
-                pot_all[q] = sum[6];
-                nnb_all[q] = (tot <= nnbmax) ? tot : -tot;
-                nbc[i] = 0;
+                double *dst = c < 3   ? acc_all + 3 * q + c
+                              : c < 6 ? jrk_all + 3 * q + (c - 3)
+                                      : pot_all + q;
+                *dst = sum;
             }
         }
-        if (lane == 0) s_tot[r] = tot;
     }
+    if (lane < niw && ib + lane < ni) {
+        nnb_all[orow(ib + lane)] = (tot <= nnbmax) ? tot : -tot;
+        nbc[ib + lane] = 0;
+    }
+    if (lane < niw) s_tot[wave * niw + lane] = tot;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        int run = 0;
-        for (int r = 0; r < ipb; ++r) {
-            const int t = s_tot[r];
-            s_off[r] = run;
-            if (t <= nnbmax) run += t;
+    if (wave == 0) {
+        // Exclusive scan of the list lengths (overflowed lists take none).
+        const int t = lane < ipb ? s_tot[lane] : 0;
+        const int len = t <= nnbmax ? t : 0;
+        int run = len;
+#pragma unroll
+        for (int o = 1; o < kP2I; o <<= 1) {
+            const int y = __shfl_up(run, o);
+            if (lane >= o) run += y;
         }
-        int base = run > 0 ? atomicAdd(total, run) : 0;
-        if ((long long)base + run > list_cap) {
-            atomicOr(err, ERR_LIST_CAP);
-            base = -1;
-        }
-        for (int r = 0; r < ipb; ++r)
-            s_off[r] = (base < 0 || s_tot[r] > nnbmax) ? -1 : base + s_off[r];
+        const int all = __builtin_amdgcn_readlane(run, kP2I - 1);
+        int base = 0;
+        if (lane == 0 && all > 0) base = atomicAdd(total, all);
+        base = __builtin_amdgcn_readfirstlane(base);
+        const bool full = (long long)base + all > list_cap;
+        if (full && lane == 0) atomicOr(err, ERR_LIST_CAP);
+        if (lane < ipb)
+            s_off[lane] = (full || t > nnbmax) ? -1 : base + run - len;
     }
+#pragma unroll
+    for (int r = 0; r < kP2W; ++r)
+        jj[r] = ent[r] < 0 ? INT_MAX : jidx ? jidx[ent[r]] : ent[r];
     __syncthreads();
 
-    int *__restrict__ row = s_rows + wave * sortcap;
-    for (int r = wave; r < ipb; r += 4) {
-        const int i = i0 + r;
-        if (i >= ni) break;
-        const int o = s_off[r];
-        int bestj = -1;
-        if (o >= 0) {
-            const int n = s_tot[r];
-            const int *__restrict__ ent = nbl + (size_t)i * cap;
-            const double xa = xi[3 * (size_t)i + 0];
-            const double ya = xi[3 * (size_t)i + 1];
-            const double za = xi[3 * (size_t)i + 2];
-            double br2 = INFINITY;
-            int bj = INT_MAX;
-            for (int e = lane; e < n; e += 64) {
-                const int p = ent[e];
-                const int j = jidx ? jidx[p] : p;
-                row[e] = j;
-                // The nearest neighbour only when the caller asks for it:
-                // it costs a record gather per list entry.
-                if (nnid_all) {
+    int off = -1, best = -1;
+    if (lane < niw) off = s_off[wave * niw + lane];
+    int *__restrict__ rows = s_rows + wave * sortcap;
+
+    // Short lists: one entry per lane, a row of 64 each.
+#pragma unroll
+    for (int r = 0; r < kP2W; ++r) rows[64 * r + lane] = jj[r];
+    __threadfence_block();
+#pragma unroll
+    for (int r = 0; r < kP2W; ++r) {
+        const int n = __builtin_amdgcn_readlane(tot, r);
+        const int o = __builtin_amdgcn_readlane(off, r);
+        if (o < 0 || n > 64) continue;
+        const int below = row_below(rows + 64 * r, n, jj[r]);
+        if (lane < n) list[o + below] = jj[r];
+        if (NN) {
+            double r2 = INFINITY;
+            if (lane < n) {
+                const size_t q = 3 * (size_t)(ib + r);
+                const JRec &J = jps[ent[r]];
+                r2 = sq3d(J.x - xi[q], J.y - xi[q + 1], J.z - xi[q + 2]);
+                if (!(r2 > 0.0)) r2 = INFINITY;
+            }
+            const int b = wave_nearest(r2, jj[r]);
+            if (lane == r) best = b;
+        }
+    }
+
+    // Longer lists, one at a time over the wavefront's whole LDS part.
+    for (int r = 0; r < niw; ++r) {
+        const int n = __builtin_amdgcn_readlane(tot, r);
+        const int o = __builtin_amdgcn_readlane(off, r);
+        if (o < 0 || n <= 64) continue;
+        const int *__restrict__ e = nbl + (size_t)(ib + r) * cap;
+        const size_t q = 3 * (size_t)(ib + r);
+        double br2 = INFINITY;
+        int bj = INT_MAX;
+        __threadfence_block();
+        const int nc = (n + 63) >> 6;
+        for (int k = lane; k < 64 * nc; k += 64) {
+            int j = INT_MAX;
+            if (k < n) {
+                const int p = e[k];
+                j = jidx ? jidx[p] : p;
+                if (NN) {
                     const JRec &J = jps[p];
-                    const double r2 = sq3d(J.x - xa, J.y - ya, J.z - za);
+                    const double r2 =
+                        sq3d(J.x - xi[q], J.y - xi[q + 1], J.z - xi[q + 2]);
                     if (r2 > 0.0 && (r2 < br2 || (r2 == br2 && j < bj))) {
                         br2 = r2;
                         bj = j;
                     }
                 }
             }
-            // Every lane of this wave reads the whole row below: the row's
-            // LDS writes complete first (the lanes run in step).
-            __threadfence_block();
-            for (int e = lane; e < n; e += 64) {
-                const int v = row[e];
-                int rank = 0;
-                for (int k = 0; k < n; ++k) rank += row[k] < v ? 1 : 0;
-                list[o + rank] = v;
-            }
-            __threadfence_block();
-            // Lexicographic (r2, j) minimum over the wave.
-            for (int w = 32; w >= 1; w >>= 1) {
-                const double r2o = __shfl_xor(br2, w);
-                const int jo = __shfl_xor(bj, w);
-                if (r2o < br2 || (r2o == br2 && jo < bj)) {
-                    br2 = r2o;
-                    bj = jo;
-                }
-            }
-            bestj = (bj == INT_MAX) ? -1 : bj;
+            rows[k] = j;
         }
-        if (lane == 0) {
-            const size_t q = orow(i);
-            off_all[q] = o;
-            if (nnid_all) nnid_all[q] = bestj;
+        __threadfence_block();
+        // Every chunk in ascending order (the wavefront's LDS accesses are
+        // in order: a chunk is read whole before it is rewritten).
+        for (int c = 0; c < nc; ++c) {
+            const int v = rows[64 * c + lane];
+            const int m = min(64, n - 64 * c);
+            const int below = row_below(rows + 64 * c, m, v);
+            __threadfence_block();
+            if (lane < m) rows[64 * c + below] = v;
         }
+        __threadfence_block();
+        for (int c = 0; c < nc; ++c) {
+            const int v = rows[64 * c + lane];
+            int below = lane;
+            for (int d = 0; d < nc; ++d)
+                if (d != c)
+                    below += run_below(rows + 64 * d, min(64, n - 64 * d), v);
+            if (64 * c + lane < n) list[o + below] = v;
+        }
+        if (NN) {
+            const int b = wave_nearest(br2, bj);
+            if (lane == r) best = b;
+        }
+    }
+
+    if (lane < niw && ib + lane < ni) {
+        const size_t q = orow(ib + lane);
+        off_all[q] = off;
+        if (NN) nnid_all[q] = best;
     }
 }
 
@@ -1304,10 +1504,6 @@ void launch_copy_from_host(hipStream_t st, const void *src, void *dst,
                        (const uint4 *)src, (uint4 *)dst, n16, zero);
 }
 
-void launch_set_desc(hipStream_t st, ClusterDesc *d, const ClusterDesc &v) {
-    hipLaunchKernelGGL(k_set_desc, dim3(1), dim3(1), 0, st, d, v);
-}
-
 void launch_zero_int(hipStream_t st, int *p, int n) {
     if (n <= 0) return;
     hipLaunchKernelGGL(k_zero_int, dim3(cdiv(n, 256)), dim3(256), 0, st, p, n);
@@ -1325,8 +1521,8 @@ static void launch_pass1(hipStream_t st, const RegfLaunch &L, long long nblk) {
     }
     hipLaunchKernelGGL((k_regf_pass1<MFLAG, G>), dim3((unsigned)nblk),
                        dim3(64 * kP1W),
-                       0, st, L.j32, L.tiles, L.jps, L.jcl, L.desc, L.ncl,
-                       L.ntask, L.jst, L.xi, L.vi, L.h2, L.dtr, L.part, L.nbc,
+                       0, st, L.j32, L.tiles, L.jps, L.jcl, L.desc, L.one,
+                       L.ncl, L.ntask, L.jst, L.xi, L.vi, L.h2, L.dtr, L.part, L.nbc,
                        L.nbl, L.err);
 }
 
@@ -1342,7 +1538,7 @@ static void launch_pass1_f64(hipStream_t st, const RegfLaunch &L,
         return;
     }
     hipLaunchKernelGGL((k_regf_pass1_f64<MFLAG, G, NR>), dim3((unsigned)nblk),
-                       dim3(64 * kP1W), 0, st, L.jps, L.desc, L.ncl, L.ntask, L.jst,
+                       dim3(64 * kP1W), 0, st, L.jps, L.desc, L.one, L.ncl, L.ntask, L.jst,
                        L.xi, L.vi, L.h2, L.dtr, L.part, L.nbc, L.nbl, L.err);
 }
 
@@ -1377,21 +1573,22 @@ void launch_regf_pass1(hipStream_t st, const RegfLaunch &L) {
 void launch_regf_pass2(hipStream_t st, const RegfLaunch &L) {
     if (L.nblk2 <= 0) return;
     const int sortcap = pass2_sortcap(L.nnbmax);
-    hipLaunchKernelGGL(k_regf_pass2, dim3((unsigned)L.nblk2), dim3(256),
+    const auto fn = L.nnid ? k_regf_pass2<true> : k_regf_pass2<false>;
+    hipLaunchKernelGGL(fn, dim3((unsigned)L.nblk2), dim3(256),
                        4 * sortcap * sizeof(int), st, L.jps, L.jidx, L.desc,
-                       L.ncl, L.xi, L.part, L.nbc, L.nbl, L.acc, L.jrk, L.pot,
-                       L.nnb, L.nnid, L.list, L.off, L.total, L.list_cap,
-                       L.nnbmax, sortcap, L.perm, L.err);
+                       L.one, L.ncl, L.xi, L.part, L.nbc, L.nbl, L.acc, L.jrk,
+                       L.pot, L.nnb, L.nnid, L.list, L.off, L.total,
+                       L.list_cap, L.nnbmax, sortcap, L.perm, L.err);
 }
 
 int pass2_sortcap(int nnbmax) {
-    return std::max(64, (nnbmax + 64) / 64 * 64);
+    return std::max(64 * kP2W, (nnbmax + 64) / 64 * 64);
 }
 
 int pass2_ipb(int ni) {
-    // About 2048 workgroups for large calls (one list-space atomic per 16 i),
-    // one i per wavefront for small ones.
-    return std::max(4, std::min(kP2I, ni / 2048));
+    // About 4096 workgroups for large calls (one list-space atomic per 32
+    // i), one i per wavefront for small ones.
+    return ni >= 65536 ? kP2I : ni >= 32768 ? 16 : ni >= 16384 ? 8 : 4;
 }
 
 void launch_pack_p(hipStream_t st, const double *m, const double *x, int n,
