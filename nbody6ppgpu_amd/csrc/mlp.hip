@@ -23,9 +23,9 @@
 //
 // Kernels
 //   k_mlp_forward   inference; 4 waves x 16 samples per workgroup, loop.
-//   k_mlp_fwdbwd    forward + backward, per-wave gradient sums accumulated
-//                   in registers over a workgroup-strided loop, one partial
-//                   row per wave.
+//   k_mlp_fwdbwd    forward + backward, a wavefront per 16 units, gradient
+//                   sums accumulated in registers over a strided loop, one
+//                   partial row per workgroup.
 //   k_mlp_reduce    sums the partial rows in a fixed order (deterministic)
 //                   and applies Adam (or only stores the sum).
 #include <hip/hip_runtime.h>
@@ -51,6 +51,11 @@ constexpr int NI = 8, NH = 64;
 constexpr int OW1 = 0, OB1 = OW1 + NH * NI, OW2 = OB1 + NH,
               OB2 = OW2 + NH * NH, OW3 = OB2 + NH, OB3 = OW3 + NH,
               NP = OB3 + 1;
+// The BF16 copy also holds W2 transposed, WT[a][b] = W2[b][a], so that every
+// MFMA operand is four consecutive values: one 8-byte load.
+constexpr int OWT = (NP + 7) / 8 * 8, NWH = OWT + NH * NH;
+static_assert(OB1 % 4 == 0 && OW2 % 4 == 0 && OB2 % 4 == 0 && OW3 % 4 == 0,
+              "8-byte operand loads");
 constexpr int kWaves = 4;               // waves per workgroup
 constexpr int kGroup = 16 * kWaves;     // samples per workgroup iteration
 constexpr int kMaxBlocks = 256;         // training workgroups (partial rows / 4)
@@ -95,26 +100,29 @@ struct FwdWeights {
     float b1[4][4], b2[4][4], w3[4][4], b3;
 };
 
+__device__ inline bf16x4 load4(const uint16_t *__restrict__ p) {
+    return *reinterpret_cast<const bf16x4 *>(p);
+}
+__device__ inline void load4f(const uint16_t *__restrict__ p, float *v) {
+    const bf16x4 h = load4(p);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = bf16_val((uint16_t)h[k]);
+}
+
 __device__ inline void load_fwd(const uint16_t *__restrict__ wh, int l,
                                 FwdWeights &W) {
     const int r = l & 15, q = l >> 4;
 #pragma unroll
     for (int T = 0; T < 4; ++T) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            W.w1[T][j] = q < 2 ? (short)wh[OW1 + (16 * T + r) * NI + 4 * q + j] : 0;
+        const bf16x4 none = {0, 0, 0, 0};
+        W.w1[T] = q < 2 ? load4(wh + OW1 + (16 * T + r) * NI + 4 * q) : none;
 #pragma unroll
         for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                W.w2[T][t][j] = (short)wh[OW2 + (16 * T + r) * NH + 16 * t + 4 * q + j];
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int u = 16 * T + 4 * q + v;
-            W.b1[T][v] = bf16_val(wh[OB1 + u]);
-            W.b2[T][v] = bf16_val(wh[OB2 + u]);
-            W.w3[T][v] = bf16_val(wh[OW3 + u]);
-        }
+            W.w2[T][t] = load4(wh + OW2 + (16 * T + r) * NH + 16 * t + 4 * q);
+        const int u = 16 * T + 4 * q;
+        load4f(wh + OB1 + u, W.b1[T]);
+        load4f(wh + OB2 + u, W.b2[T]);
+        load4f(wh + OW3 + u, W.w3[T]);
     }
     W.b3 = bf16_val(wh[OB3]);
 }
@@ -138,22 +146,17 @@ __device__ inline bf16x4 input_operand(const Norm &nm, const float *__restrict__
     return b;
 }
 
-// Forward of the wave's 16 samples.  Outputs (result layout, lane = sample
-// l%16, units 16T+4q+v): h1 as the layer-2 B operands, silu'(z1), h2,
-// silu'(z2); returns the network output for sample l%16 (in every lane).
-__device__ inline float forward16(const FwdWeights &W, bf16x4 xb, bf16x4 *h1b,
-                                  float (*ds1)[4], float (*h2)[4],
-                                  float (*ds2)[4]) {
+// Forward of the wave's 16 samples (result layout: lane = sample l%16, units
+// 16T+4q+v): the network output for sample l%16, in every lane.
+__device__ inline float forward16(const FwdWeights &W, bf16x4 xb) {
     const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    bf16x4 h1b[4];
 #pragma unroll
     for (int T = 0; T < 4; ++T) {
         const f32x4 z = mfma16(W.w1[T], xb, zero);
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const float zz = z[v] + W.b1[T][v];
-            h1b[T][v] = (short)bf16_bits(silu(zz));
-            if (ds1) ds1[T][v] = dsilu(zz);
-        }
+        for (int v = 0; v < 4; ++v)
+            h1b[T][v] = (short)bf16_bits(silu(z[v] + W.b1[T][v]));
     }
     float part = 0.0f;
 #pragma unroll
@@ -163,10 +166,7 @@ __device__ inline float forward16(const FwdWeights &W, bf16x4 xb, bf16x4 *h1b,
         for (int t = 0; t < 4; ++t) z = mfma16(W.w2[T][t], h1b[t], z);
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const float zz = z[v] + W.b2[T][v];
-            const float h = bf16_val(bf16_bits(silu(zz)));
-            if (h2) h2[T][v] = h;
-            if (ds2) ds2[T][v] = dsilu(zz);
+            const float h = bf16_val(bf16_bits(silu(z[v] + W.b2[T][v])));
             part = fmaf(W.w3[T][v], h, part);
         }
     }
@@ -189,8 +189,7 @@ __global__ __launch_bounds__(256) void k_mlp_forward(
         const bool valid = sidx < n;
         float xh[4];
         const bf16x4 xb = input_operand(nm, x, sidx, valid, q, xh);
-        bf16x4 h1b[4];
-        const float out = forward16(W, xb, h1b, nullptr, nullptr, nullptr);
+        const float out = forward16(W, xb);
         if (valid && q == 0) y[sidx] = out * nm.ys + nm.ym;
     }
 }
@@ -199,177 +198,251 @@ __global__ __launch_bounds__(256) void k_mlp_forward(
 // identity).  Loss = mean over the batch of (yhat - t_normalised)^2.  The
 // derivative of the BF16 rounding is taken as 1 (straight-through).  Deltas
 // d2 and d1 enter the MFMA products (d1 = W2^T d2, the weight gradients) as
-// BF16; the bias and output-layer gradients use them in FP32.  Each wave
-// accumulates its gradient sums over its samples and writes them, with its
-// summed squared error, to row blockIdx.x*kWaves + wave of gpart / lpart.
+// BF16; the bias and output-layer gradients use them in FP32.
+//
+// Workgroup b accumulates partial row b: the 16-sample groups b % 4 of the
+// 64-sample blocks b / 4, b / 4 + gridDim / 4, ... in turn.  Its four
+// wavefronts split a group by units: wavefront T evaluates units 16T..16T+15
+// of every layer (an MFMA tile) and passes activations and deltas to the
+// others through LDS.  A minibatch of 1024 has only 64 groups, and a
+// wavefront alone on its SIMD issues an instruction every 7-8 cycles, so the
+// length of a wavefront's instruction stream is the kernel's time: 16 us with
+// a group per wavefront, 7 us so.
 constexpr int LDS_ROW = NH + 8;   // bf16 per sample row (16-byte padding)
+static_assert(NH == 16 * kWaves, "a wavefront per tile of units");
 __global__ __launch_bounds__(256) void k_mlp_fwdbwd(
     int count, int base, const int *__restrict__ idx,
     const float *__restrict__ x, const float *__restrict__ t,
     const uint16_t *__restrict__ wh, Norm nm, float inv_batch,
     float *__restrict__ gpart, float *__restrict__ lpart) {
-    __shared__ uint16_t sH1[kWaves][16 * LDS_ROW];
-    __shared__ uint16_t sD2[kWaves][16 * LDS_ROW];
-    __shared__ uint16_t sD1[kWaves][16 * LDS_ROW];
-    __shared__ uint16_t sXH[kWaves][16 * 16];
-    const int l = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    __shared__ __align__(16) uint16_t h1s[16 * LDS_ROW], h2s[16 * LDS_ROW];
+    __shared__ __align__(16) uint16_t d2s[16 * LDS_ROW], d1s[16 * LDS_ROW];
+    __shared__ uint16_t xs[16 * 16];
+    const int l = threadIdx.x & 63;
+    const int T = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = l & 15, q = l >> 4;
-    FwdWeights W;
-    load_fwd(wh, l, W);
-    // A operand of d1^T = W2^T d2^T: lane holds W2[16t+4q+j][16T+r].
-    bf16x4 w2t[4][4];
+    const int u0 = 16 * T + 4 * q;    // this lane's units of a result tile
+    // Operands of this wavefront's tile (see FwdWeights), and of d1^T = W2^T
+    // d2^T: lane holds W2[16t+4q+j][16T+r].
+    const bf16x4 none = {0, 0, 0, 0};
+    const bf16x4 w1 = q < 2 ? load4(wh + OW1 + (16 * T + r) * NI + 4 * q) : none;
+    bf16x4 w2[4], w2t[4];
+    float b1[4], b2[4], w3[4], w3all[4][4];
 #pragma unroll
-    for (int T = 0; T < 4; ++T)
-#pragma unroll
-        for (int tt = 0; tt < 4; ++tt)
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                w2t[T][tt][j] = (short)wh[OW2 + (16 * tt + 4 * q + j) * NH + 16 * T + r];
-    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-    f32x4 gw2[4][4], gw1[4];
-    float gb1[4][4], gb2[4][4], gw3[4][4], gb3 = 0.0f, loss = 0.0f;
-#pragma unroll
-    for (int T = 0; T < 4; ++T) {
-        gw1[T] = zero;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            gw2[T][v] = zero;
-            gb1[T][v] = gb2[T][v] = gw3[T][v] = 0.0f;
-        }
+    for (int k = 0; k < 4; ++k) {
+        w2[k] = load4(wh + OW2 + (16 * T + r) * NH + 16 * k + 4 * q);
+        w2t[k] = load4(wh + OWT + (16 * T + r) * NH + 16 * k + 4 * q);
+        load4f(wh + OW3 + 16 * k + 4 * q, w3all[k]);
     }
-    uint16_t *h1s = sH1[wave], *d2s = sD2[wave], *d1s = sD1[wave], *xs = sXH[wave];
+    load4f(wh + OB1 + u0, b1);
+    load4f(wh + OB2 + u0, b2);
+    load4f(wh + OW3 + u0, w3);
+    const float b3 = bf16_val(wh[OB3]);
+    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    f32x4 gw2[4], gw1 = zero;
+    float gb1[4], gb2[4], gw3[4], gb3 = 0.0f, loss = 0.0f;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        gw2[v] = zero;
+        gb1[v] = gb2[v] = gw3[v] = 0.0f;
+    }
+    const int row = r * LDS_ROW;      // this lane's sample
     const int nbg = (count + kGroup - 1) / kGroup;
     // Uniform trip count across the workgroup (barriers inside the loop).
-    for (int bg = blockIdx.x; bg < nbg; bg += gridDim.x) {
-        const int qi = bg * kGroup + 16 * wave + r;
+    for (int bg = blockIdx.x / kWaves; bg < nbg; bg += gridDim.x / kWaves) {
+        const int qi = bg * kGroup + 16 * (int)(blockIdx.x % kWaves) + r;
         const bool valid = qi < count;
         const int sidx = valid ? (idx ? idx[base + qi] : base + qi) : 0;
         float xh[4];
         const bf16x4 xb = input_operand(nm, x, sidx, valid, q, xh);
-        bf16x4 h1b[4];
-        float ds1[4][4], h2[4][4], ds2[4][4];
-        const float out = forward16(W, xb, h1b, ds1, h2, ds2);
+        const float tn = valid ? (t[sidx] - nm.ym) / nm.ys : 0.0f;
+        bf16x4 hb;
+        float ds1[4], ds2[4], h2[4];
+        f32x4 z = mfma16(w1, xb, zero);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const float zz = z[v] + b1[v];
+            hb[v] = (short)bf16_bits(silu(zz));
+            ds1[v] = dsilu(zz);
+        }
+        *reinterpret_cast<bf16x4 *>(h1s + row + u0) = hb;
+        __syncthreads();
+        z = zero;
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            z = mfma16(w2[k], load4(h1s + row + 16 * k + 4 * q), z);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const float zz = z[v] + b2[v];
+            hb[v] = (short)bf16_bits(silu(zz));
+            h2[v] = bf16_val((uint16_t)hb[v]);
+            ds2[v] = dsilu(zz);
+        }
+        *reinterpret_cast<bf16x4 *>(h2s + row + u0) = hb;
+        __syncthreads();
+        // The output, in every wavefront: the lane's units of all tiles in
+        // order, then the four lanes holding this sample (as in forward16).
+        float part = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const bf16x4 h = load4(h2s + row + 16 * k + 4 * q);
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                part = fmaf(w3all[k][v], bf16_val((uint16_t)h[v]), part);
+        }
+        part += __shfl_xor(part, 16);
+        part += __shfl_xor(part, 32);
+        const float out = part + b3;
         float d3 = 0.0f;
         if (valid) {
-            const float e = out - (t[sidx] - nm.ym) / nm.ys;
+            const float e = out - tn;
             d3 = 2.0f * e * inv_batch;
             if (q == 0) loss += e * e;
         }
         if (q == 0) gb3 += d3;
         // d2 (result layout of layer 2 = B operand of the d1 product).
-        bf16x4 d2b[4];
+        bf16x4 db;
 #pragma unroll
-        for (int T = 0; T < 4; ++T)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const float d2 = d3 * W.w3[T][v] * ds2[T][v];
-                d2b[T][v] = (short)bf16_bits(d2);
-                gb2[T][v] += d2;
-                gw3[T][v] = fmaf(d3, h2[T][v], gw3[T][v]);
-            }
-        // d1^T = W2^T d2^T, then times silu'(z1).
-#pragma unroll
-        for (int T = 0; T < 4; ++T) {
-            f32x4 z = zero;
-#pragma unroll
-            for (int tt = 0; tt < 4; ++tt) z = mfma16(w2t[T][tt], d2b[tt], z);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const float d1 = z[v] * ds1[T][v];
-                gb1[T][v] += d1;
-                const int u = 16 * T + 4 * q + v;
-                d1s[r * LDS_ROW + u] = bf16_bits(d1);
-                d2s[r * LDS_ROW + u] = (uint16_t)d2b[T][v];
-                h1s[r * LDS_ROW + u] = (uint16_t)h1b[T][v];
-            }
+        for (int v = 0; v < 4; ++v) {
+            const float d2 = d3 * w3[v] * ds2[v];
+            db[v] = (short)bf16_bits(d2);
+            gb2[v] += d2;
+            gw3[v] = fmaf(d3, h2[v], gw3[v]);
         }
+        *reinterpret_cast<bf16x4 *>(d2s + row + u0) = db;
+        __syncthreads();
+        // d1^T = W2^T d2^T, then times silu'(z1).
+        z = zero;
 #pragma unroll
-        for (int v = 0; v < 4; ++v)
-            xs[r * 16 + 4 * q + v] = q < 2 ? bf16_bits(xh[v]) : 0;
+        for (int k = 0; k < 4; ++k)
+            z = mfma16(w2t[k], load4(d2s + row + 16 * k + 4 * q), z);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const float d1 = z[v] * ds1[v];
+            gb1[v] += d1;
+            db[v] = (short)bf16_bits(d1);
+        }
+        *reinterpret_cast<bf16x4 *>(d1s + row + u0) = db;
+        if (T == 0) {
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                xs[r * 16 + 4 * q + v] = q < 2 ? bf16_bits(xh[v]) : 0;
+        }
         __syncthreads();
         // Weight gradients: samples on the k dimension.
         //   gW2[b][a] += sum_s d2[s][b] h1[s][a]:  A[b][s], B[s][a]
         //   gW1[a][k] += sum_s d1[s][a] xh[s][k]:  A[a][s], B[s][k]
-        bf16x4 ad2[4], ad1[4], bh1[4], bx;
+        bf16x4 ad2, ad1, bh1[4], bx;
 #pragma unroll
-        for (int T = 0; T < 4; ++T)
+        for (int j = 0; j < 4; ++j) {
+            const int at = (4 * q + j) * LDS_ROW;
+            ad2[j] = (short)d2s[at + 16 * T + r];
+            ad1[j] = (short)d1s[at + 16 * T + r];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int row = (4 * q + j) * LDS_ROW + 16 * T + r;
-                ad2[T][j] = (short)d2s[row];
-                ad1[T][j] = (short)d1s[row];
-                bh1[T][j] = (short)h1s[row];
-            }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) bx[j] = (short)xs[(4 * q + j) * 16 + r];
-#pragma unroll
-        for (int T = 0; T < 4; ++T) {
-#pragma unroll
-            for (int T2 = 0; T2 < 4; ++T2) gw2[T][T2] = mfma16(ad2[T], bh1[T2], gw2[T][T2]);
-            gw1[T] = mfma16(ad1[T], bx, gw1[T]);
+            for (int k = 0; k < 4; ++k) bh1[k][j] = (short)h1s[at + 16 * k + r];
+            bx[j] = (short)xs[(4 * q + j) * 16 + r];
         }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) gw2[k] = mfma16(ad2, bh1[k], gw2[k]);
+        gw1 = mfma16(ad1, bx, gw1);
         __syncthreads();
     }
-    // Partial row of this wave.
-    float *g = gpart + (size_t)(blockIdx.x * kWaves + wave) * NP;
+    // This wavefront's units of the partial row.
+    float *g = gpart + (size_t)blockIdx.x * NP;
 #pragma unroll
-    for (int T = 0; T < 4; ++T)
+    for (int v = 0; v < 4; ++v) {
+        const int u = u0 + v;   // row unit of the result tiles
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int u = 16 * T + 4 * q + v;   // row unit of the result tiles
+        for (int k = 0; k < 4; ++k) g[OW2 + u * NH + 16 * k + r] = gw2[k][v];
+        if (r < NI) g[OW1 + u * NI + r] = gw1[v];
+        // Bias / output-layer sums over the 16 samples of this lane group.
+        float a1 = gb1[v], a2 = gb2[v], a3 = gw3[v];
 #pragma unroll
-            for (int T2 = 0; T2 < 4; ++T2) g[OW2 + u * NH + 16 * T2 + r] = gw2[T][T2][v];
-            if (r < NI) g[OW1 + u * NI + r] = gw1[T][v];
-            // Bias / output-layer sums over the 16 samples of this lane group.
-            float a1 = gb1[T][v], a2 = gb2[T][v], a3 = gw3[T][v];
-#pragma unroll
-            for (int o = 1; o < 16; o <<= 1) {
-                a1 += __shfl_xor(a1, o);
-                a2 += __shfl_xor(a2, o);
-                a3 += __shfl_xor(a3, o);
-            }
-            if (r == 0) {
-                g[OB1 + u] = a1;
-                g[OB2 + u] = a2;
-                g[OW3 + u] = a3;
-            }
+        for (int o = 1; o < 16; o <<= 1) {
+            a1 += __shfl_xor(a1, o);
+            a2 += __shfl_xor(a2, o);
+            a3 += __shfl_xor(a3, o);
         }
+        if (r == 0) {
+            g[OB1 + u] = a1;
+            g[OB2 + u] = a2;
+            g[OW3 + u] = a3;
+        }
+    }
+    if (T != 0) return;
     for (int o = 32; o >= 1; o >>= 1) {
         gb3 += __shfl_xor(gb3, o);
         loss += __shfl_xor(loss, o);
     }
     if (l == 0) {
         g[OB3] = gb3;
-        lpart[blockIdx.x * kWaves + wave] = loss;
+        lpart[blockIdx.x] = loss;
+    }
+}
+
+// BF16 copy of parameter k (and its place in WT).
+__device__ inline void store_bf16(uint16_t *__restrict__ wh, int k, float w) {
+    const uint16_t h = bf16_bits(w);
+    wh[k] = h;
+    if (k >= OW2 && k < OB2) {
+        const int b = (k - OW2) / NH, a = (k - OW2) % NH;
+        wh[OWT + a * NH + b] = h;
     }
 }
 
 // Sum the nrow partial rows in row order; with adam != 0 apply one Adam step
-// to the FP32 masters and refresh the BF16 copy.
-__global__ __launch_bounds__(256) void k_mlp_reduce(
+// to the FP32 masters and refresh the BF16 copy.  One wavefront per 64
+// parameters; kRedU rows are loaded together and added in order (a row at a
+// time, the kernel was one memory round trip per few rows: 64 rows 17 us,
+// now 4 us).
+constexpr int kRedU = 32;
+__global__ __launch_bounds__(64) void k_mlp_reduce(
     int nrow, const float *__restrict__ gpart, float *__restrict__ gsum,
     int adam, float lr, float b1, float b2, float eps, float c1, float c2,
     float *__restrict__ w, uint16_t *__restrict__ wh, float *__restrict__ m,
     float *__restrict__ v) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= NP) return;
+    float m0 = 0.0f, v0 = 0.0f, w0 = 0.0f;
+    if (adam) {
+        m0 = m[k];
+        v0 = v[k];
+        w0 = w[k];
+    }
     float g = 0.0f;
-    for (int b = 0; b < nrow; ++b) g += gpart[(size_t)b * NP + k];
+    const float *__restrict__ p = gpart + k;
+    int b = 0;
+    for (; b + kRedU <= nrow; b += kRedU) {
+        float r[kRedU];
+#pragma unroll
+        for (int u = 0; u < kRedU; ++u) r[u] = p[(size_t)(b + u) * NP];
+#pragma unroll
+        for (int u = 0; u < kRedU; ++u) g += r[u];
+    }
+    if (b < nrow) {
+        float r[kRedU];
+#pragma unroll
+        for (int u = 0; u < kRedU; ++u)
+            r[u] = b + u < nrow ? p[(size_t)(b + u) * NP] : 0.0f;
+#pragma unroll
+        for (int u = 0; u < kRedU; ++u)
+            if (b + u < nrow) g += r[u];
+    }
     gsum[k] = g;
     if (adam) {
-        const float mk = b1 * m[k] + (1.0f - b1) * g;
-        const float vk = b2 * v[k] + (1.0f - b2) * g * g;
+        const float mk = b1 * m0 + (1.0f - b1) * g;
+        const float vk = b2 * v0 + (1.0f - b2) * g * g;
         m[k] = mk;
         v[k] = vk;
-        const float wk = w[k] - lr * (mk / c1) / (sqrtf(vk / c2) + eps);
+        const float wk = w0 - lr * (mk / c1) / (sqrtf(vk / c2) + eps);
         w[k] = wk;
-        wh[k] = bf16_bits(wk);
+        store_bf16(wh, k, wk);
     }
 }
 
 __global__ void k_bf16_copy(const float *__restrict__ w, uint16_t *__restrict__ wh) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < NP) wh[k] = bf16_bits(w[k]);
+    if (k < NP) store_bf16(wh, k, w[k]);
 }
 
 // ---------------------------------------------------------------------------
@@ -388,7 +461,7 @@ struct State {
     float *dx = nullptr, *dt = nullptr, *dy = nullptr, *gpart = nullptr,
           *lpart = nullptr;
     int *didx = nullptr;
-    size_t cap_n = 0, cap_rows = 0;
+    size_t cap_n = 0, cap_rows = 0, cap_loss = 0;
 };
 State M;
 
@@ -404,7 +477,7 @@ void ensure_init() {
     if (M.init) return;
     MCHK(hipStreamCreateWithFlags(&M.st, hipStreamNonBlocking));
     MCHK(hipMalloc((void **)&M.w, NP * sizeof(float)));
-    MCHK(hipMalloc((void **)&M.wh, NP * sizeof(uint16_t)));
+    MCHK(hipMalloc((void **)&M.wh, NWH * sizeof(uint16_t)));
     MCHK(hipMalloc((void **)&M.m, NP * sizeof(float)));
     MCHK(hipMalloc((void **)&M.v, NP * sizeof(float)));
     MCHK(hipMalloc((void **)&M.gsum, NP * sizeof(float)));
@@ -417,7 +490,8 @@ void ensure_init() {
     M.init = true;
 }
 
-void ensure_data(size_t n, size_t nrows) {
+// Samples, partial gradient rows and partial losses the buffers hold.
+void ensure_data(size_t n, size_t nrows, size_t nloss) {
     if (n > M.cap_n) {
         if (M.dx) (void)hipFree(M.dx);
         if (M.dt) (void)hipFree(M.dt);
@@ -431,10 +505,17 @@ void ensure_data(size_t n, size_t nrows) {
     }
     if (nrows > M.cap_rows) {
         if (M.gpart) (void)hipFree(M.gpart);
-        if (M.lpart) (void)hipFree(M.lpart);
+        M.gpart = nullptr;
+        M.cap_rows = 0;
         MCHK(hipMalloc((void **)&M.gpart, nrows * NP * sizeof(float)));
-        MCHK(hipMalloc((void **)&M.lpart, nrows * sizeof(float)));
         M.cap_rows = nrows;
+    }
+    if (nloss > M.cap_loss) {
+        if (M.lpart) (void)hipFree(M.lpart);
+        M.lpart = nullptr;
+        M.cap_loss = 0;
+        MCHK(hipMalloc((void **)&M.lpart, nloss * sizeof(float)));
+        M.cap_loss = nloss;
     }
 }
 
@@ -449,16 +530,21 @@ void set_params(const float *p) {
     M.adam_t = 0;
 }
 
-// One pass of forward+backward over count samples starting at base (through
-// idx if given); gradient (mean-square loss) summed into M.gsum, optionally
-// followed by an Adam step.  Returns the summed squared error.
-double grad_step(int count, int base, const int *didx, float lr, int adam) {
-    const int nblk = std::min((count + kGroup - 1) / kGroup, kMaxBlocks);
-    const int nrows = nblk * kWaves;
-    ensure_data(M.cap_n, (size_t)nrows);
-    hipLaunchKernelGGL(k_mlp_fwdbwd, dim3(nblk), dim3(64 * kWaves), 0, M.st,
-                       count, base, didx, M.dx, M.dt, M.wh, M.nm,
-                       1.0f / count, M.gpart, M.lpart);
+// Partial rows (one per workgroup) of a pass over count samples.
+int rows_of(int count) {
+    return std::min((count + kGroup - 1) / kGroup, kMaxBlocks) * kWaves;
+}
+
+// Enqueue one pass of forward+backward over count samples starting at base
+// (through idx if given): gradient (mean-square loss) summed into M.gsum,
+// optionally followed by an Adam step, and the summed squared errors of its
+// rows_of(count) rows in lpart.
+void grad_step(int count, int base, const int *didx, float lr, int adam,
+               float *lpart) {
+    const int nrows = rows_of(count);
+    hipLaunchKernelGGL(k_mlp_fwdbwd, dim3(nrows), dim3(64 * kWaves), 0,
+                       M.st, count, base, didx, M.dx, M.dt, M.wh, M.nm,
+                       1.0f / count, M.gpart, lpart);
     float c1 = 1.0f, c2 = 1.0f;
     const float b1 = 0.9f, b2 = 0.999f;
     if (adam) {
@@ -466,22 +552,22 @@ double grad_step(int count, int base, const int *didx, float lr, int adam) {
         c1 = 1.0f - std::pow(b1, (float)M.adam_t);
         c2 = 1.0f - std::pow(b2, (float)M.adam_t);
     }
-    hipLaunchKernelGGL(k_mlp_reduce, dim3((NP + 255) / 256), dim3(256), 0,
+    hipLaunchKernelGGL(k_mlp_reduce, dim3((NP + 63) / 64), dim3(64), 0,
                        M.st, nrows, M.gpart, M.gsum, adam, lr, b1, b2, 1e-8f,
                        c1, c2, M.w, M.wh, M.m, M.v);
     MCHK(hipGetLastError());
-    std::vector<float> lp(nrows);
-    MCHK(hipMemcpyAsync(lp.data(), M.lpart, nrows * sizeof(float),
-                        hipMemcpyDeviceToHost, M.st));
-    MCHK(hipStreamSynchronize(M.st));
+}
+
+// The summed squared error of one pass from its rows' sums.
+double loss_sum(const float *lp, int nrows) {
     double l = 0.0;
-    for (float q : lp) l += q;
+    for (int k = 0; k < nrows; ++k) l += lp[k];
     return l;
 }
 
 void upload_data(int n, const float *x, const float *t) {
     ensure_init();
-    ensure_data((size_t)n, 1);
+    ensure_data((size_t)n, 0, 0);
     MCHK(hipMemcpyAsync(M.dx, x, (size_t)n * NI * sizeof(float),
                         hipMemcpyHostToDevice, M.st));
     if (t)
@@ -563,11 +649,16 @@ MLP_EXPORT int gpunb_mlp_grad(int n, const float *x, const float *t,
     return gpunb::run_guarded("gpunb_mlp_grad", [&] {
         if (n <= 0) throw std::runtime_error("n must be > 0");
         upload_data(n, x, t);
-        const double l = grad_step(n, 0, nullptr, 0.0f, 0);
+        const int nrows = rows_of(n);
+        ensure_data(0, (size_t)nrows, (size_t)nrows);
+        grad_step(n, 0, nullptr, 0.0f, 0, M.lpart);
+        std::vector<float> lp(nrows);
+        MCHK(hipMemcpyAsync(lp.data(), M.lpart, nrows * sizeof(float),
+                            hipMemcpyDeviceToHost, M.st));
         MCHK(hipMemcpyAsync(grad, M.gsum, NP * sizeof(float),
                             hipMemcpyDeviceToHost, M.st));
         MCHK(hipStreamSynchronize(M.st));
-        if (loss) *loss = l / n;
+        if (loss) *loss = loss_sum(lp.data(), nrows) / n;
     });
 }
 
@@ -577,23 +668,36 @@ MLP_EXPORT int gpunb_mlp_train(int n, const float *x, const float *t,
     return gpunb::run_guarded("gpunb_mlp_train", [&] {
         if (n <= 0 || epochs <= 0 || batch <= 0)
             throw std::runtime_error("n, epochs and batch must be > 0");
+        // The whole epoch is enqueued at once: the minibatches' losses stay on
+        // the device (row_max partial sums each) until the last epoch is done.
+        const int nb = (n - 1) / batch + 1;
+        const int row_max = rows_of(std::min(batch, n));
         upload_data(n, x, t);
+        ensure_data(0, (size_t)row_max, (size_t)nb * row_max);
         std::vector<int> idx(n);
         for (int k = 0; k < n; ++k) idx[k] = k;
         std::mt19937 rng(seed);
-        double last = 0.0;
         for (int e = 0; e < epochs; ++e) {
             std::shuffle(idx.begin(), idx.end(), rng);
-            MCHK(hipMemcpyAsync(M.didx, idx.data(), (size_t)n * sizeof(int),
-                                hipMemcpyHostToDevice, M.st));
-            double sum = 0.0;
-            for (int b0 = 0; b0 < n; b0 += batch) {
-                const int cnt = std::min(batch, n - b0);
-                sum += grad_step(cnt, b0, M.didx, lr, 1);
+            // Synchronous, so that idx may be shuffled again; in stream order
+            // behind the previous epoch, which reads the old order.
+            MCHK(hipMemcpyWithStream(M.didx, idx.data(), (size_t)n * sizeof(int),
+                                     hipMemcpyHostToDevice, M.st));
+            for (int b = 0; b < nb; ++b) {
+                const int b0 = b * batch;
+                grad_step(std::min(batch, n - b0), b0, M.didx, lr, 1,
+                          M.lpart + (size_t)b * row_max);
             }
-            last = sum / n;
         }
-        if (loss_out) *loss_out = last;
+        std::vector<float> lp((size_t)nb * row_max);
+        MCHK(hipMemcpyAsync(lp.data(), M.lpart, lp.size() * sizeof(float),
+                            hipMemcpyDeviceToHost, M.st));
+        MCHK(hipStreamSynchronize(M.st));
+        double sum = 0.0;
+        for (int b = 0; b < nb; ++b)
+            sum += loss_sum(lp.data() + (size_t)b * row_max,
+                            rows_of(std::min(batch, n - b * batch)));
+        if (loss_out) *loss_out = sum / n;
     });
 }
 
