@@ -246,6 +246,7 @@ struct State {
     long long list_est = 0;
 
     DevBuf<PRec> pot_rec;
+    DevBuf<float> pot_m;
     DevBuf<double> d_pin, d_ppart, d_pout;
     HostBuf<double> h_pin, h_pout;
 
@@ -1012,6 +1013,34 @@ void do_profile(int irank) {
     S.icall = S.ini = S.isend = 0;
 }
 
+// Potential of bodies i0 .. i0 + ni - 1 over all n, device arrays.  All
+// bodies of a set of 4096 to 4M go through the kernel that forms each 1/r
+// once (its partials are 2 KiB a body at the upper end); below, its block
+// pairs would not fill the machine (N = 4096: 63 us a call, 67 with
+// k_pot_pass1; N = 16384: 143 and 167; N = 131072: 3.59 and 5.83 ms).
+void enqueue_pot(const double *d_m, const double *d_x, int n, int i0, int ni,
+                 double *d_pot) {
+    const int ntile = cdiv(n, kTile);
+    const size_t n_pad = (size_t)ntile * kTile;
+    S.pot_rec.ensure(n_pad + kTile);
+    S.pot_m.ensure(n_pad + kTile);
+    launch_pack_p(S.st, d_m, d_x, n, (int)n_pad + kTile, S.pot_rec.p, S.pot_m.p,
+                  S.err.p);
+    if (i0 == 0 && ni == n && n >= 4096 && n <= (1 << 22)) {
+        const PotSym P = pot_sym_plan(ntile);
+        S.d_ppart.ensure((size_t)(P.nblock + 1) * n_pad);
+        launch_pot_sym(S.st, S.pot_rec.p, S.pot_m.p, n, ntile, P, S.d_ppart.p,
+                       d_pot);
+        return;
+    }
+    if (!S.pot_resident) S.pot_resident = pot_resident_waves();
+    const int target = std::max(S.pot_resident, 1024) * 2;
+    int ns = std::max(1, (int)std::lround((double)target / cdiv(ni, 64)));
+    ns = std::min(ns, std::max(ntile, 1));
+    S.d_ppart.ensure((size_t)round_up(ni, 64) * ns);
+    launch_pot(S.st, S.pot_rec.p, ntile, i0, ni, ns, S.d_ppart.p, d_pot);
+}
+
 void do_pot(int irank, int istart, int ni, int n, const double *m,
             const double (*x)[3], double *pot) {
     devinit(irank);
@@ -1021,27 +1050,15 @@ void do_pot(int irank, int istart, int ni, int n, const double *m,
     if (ni == 0) return;
     double t0 = wtime();
     set_device();
-    const int ntile = cdiv(n, kTile);
-    const int n_pad = ntile * kTile;
     S.h_pin.ensure(4 * (size_t)n);
     S.d_pin.ensure(4 * (size_t)n);
-    S.pot_rec.ensure((size_t)n_pad + kTile);
     memcpy(S.h_pin.p, m, (size_t)n * sizeof(double));
     memcpy(S.h_pin.p + n, x, 3 * (size_t)n * sizeof(double));
     HIPCHK(hipMemcpyAsync(S.d_pin.p, S.h_pin.p, 4 * (size_t)n * sizeof(double),
                           hipMemcpyHostToDevice, S.st));
-    launch_pack_p(S.st, S.d_pin.p, S.d_pin.p + n, n, n_pad + kTile, S.pot_rec.p,
-                  S.err.p);
-    if (!S.pot_resident) S.pot_resident = pot_resident_waves();
-    const int target = std::max(S.pot_resident, 1024) * 2;
-    const int n_iw = cdiv(ni, 64);
-    int ns = std::max(1, (int)std::lround((double)target / n_iw));
-    ns = std::min(ns, std::max(ntile, 1));
-    S.d_ppart.ensure((size_t)round_up(ni, 64) * ns);
     S.d_pout.ensure((size_t)ni);
     S.h_pout.ensure((size_t)ni);
-    launch_pot(S.st, S.pot_rec.p, n, ntile, istart - 1, ni, ns, S.d_ppart.p,
-               S.d_pout.p);
+    enqueue_pot(S.d_pin.p, S.d_pin.p + n, n, istart - 1, ni, S.d_pout.p);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(S.h_pout.p, S.d_pout.p, (size_t)ni * sizeof(double),
                           hipMemcpyDeviceToHost, S.st));
@@ -1708,20 +1725,9 @@ GPUNB_EXPORT int gpunb_energy_dev(const gpunb_energy_par *par,
         set_device();
         const int nb = P.ntot - P.ifirst + 1;
         if (run_pot && nb > 0) {
-            const int ntile = cdiv(nb, kTile);
-            const int n_pad = ntile * kTile;
-            S.pot_rec.ensure((size_t)n_pad + kTile);
-            launch_pack_p(S.st, d_body + (P.ifirst - 1),
-                          d_x + 3 * (size_t)(P.ifirst - 1), nb, n_pad + kTile,
-                          S.pot_rec.p, S.err.p);
-            if (!S.pot_resident) S.pot_resident = pot_resident_waves();
-            const int target = std::max(S.pot_resident, 1024) * 2;
-            const int n_iw = cdiv(nb, 64);
-            int ns = std::max(1, (int)std::lround((double)target / n_iw));
-            ns = std::min(ns, std::max(ntile, 1));
-            S.d_ppart.ensure((size_t)round_up(nb, 64) * ns);
-            launch_pot(S.st, S.pot_rec.p, nb, ntile, 0, nb, ns, S.d_ppart.p,
-                       d_phidbl + (P.ifirst - 1));
+            enqueue_pot(d_body + (P.ifirst - 1),
+                        d_x + 3 * (size_t)(P.ifirst - 1), nb, 0, nb,
+                        d_phidbl + (P.ifirst - 1));
         }
         S.en_cpot.ensure((size_t)std::max(nb, 1));
         S.en_ckin.ensure((size_t)std::max(nb, 1));

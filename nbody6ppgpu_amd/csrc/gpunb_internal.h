@@ -287,10 +287,22 @@ void launch_copy_to_host(hipStream_t st, const void *src, void *dst,
 // pinned host buffer to device memory, and *zero = 0.
 void launch_copy_from_host(hipStream_t st, const void *src, void *dst,
                            size_t bytes, int *zero);
-void launch_pot(hipStream_t st, const PRec *p, int n, int ntile, int i0,
-                int ni, int nslice, double *part, double *pot);
+// Potential (pot.hip).  p, pm: records and FP32 masses of the bodies padded to
+// whole tiles (mass 0, far away) plus one spare tile (launch_pack_p).
 void launch_pack_p(hipStream_t st, const double *m, const double *x, int n,
-                   int n_pad, PRec *p, unsigned *err);
+                   int n_pad, PRec *p, float *pm, unsigned *err);
+// Bodies i0 .. i0 + ni - 1 over all; part: ni rounded up to 64, times nslice.
+void launch_pot(hipStream_t st, const PRec *p, int ntile, int i0, int ni,
+                int nslice, double *part, double *pot);
+// All n bodies over all.  part: (nblock + 1) rows of ntile * kTile.
+struct PotSym {
+    int k;        // tiles held by a wavefront
+    int nsub;     // groups of k tiles per block
+    int nblock;
+};
+PotSym pot_sym_plan(int ntile);
+void launch_pot_sym(hipStream_t st, const PRec *p, const float *pm, int n,
+                    int ntile, const PotSym &P, double *part, double *pot);
 
 // One regular-corrector call (regcor.hip).
 struct RegcorLaunch {

@@ -17,7 +17,6 @@
 //   k_regf_pass1_f64  the same in FP64 throughout (_q: persistent form).
 //   k_regf_pass2   per-i FP64 reduction of the slice partials, ordered list
 //                  compaction and (when asked for) the nearest neighbour.
-//   k_pot_pass1/2  O(N^2) potential (gpupot.gpu.cu:32-57).
 #include "gpunb_internal.h"
 
 #include <algorithm>
@@ -1353,101 +1352,6 @@ __global__ __launch_bounds__(256) void k_regf_pass2(
 }
 
 // ---------------------------------------------------------------------------
-// Potential: phi_i = sum_{j: r2 > 0} m_j / r_ij.  FP64 differences, FP32
-// r2 / rsqrt / products, FP32 tile sums folded into FP64.
-// ---------------------------------------------------------------------------
-
-__global__ __launch_bounds__(256) void k_pack_p(const double *__restrict__ m,
-                                                const double *__restrict__ x,
-                                                int n, int n_pad,
-                                                PRec *__restrict__ p,
-                                                unsigned *__restrict__ err) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j < n) {
-        PRec r;
-        r.x = x[3 * (size_t)j + 0];
-        r.y = x[3 * (size_t)j + 1];
-        r.z = x[3 * (size_t)j + 2];
-        const double mj = m[j];
-        r.m32 = (float)mj;
-        r.pad = 0.0f;
-        const double chk = r.x + r.y + r.z + mj;
-        if (chk != chk) atomicOr(err, ERR_NAN_J);
-        p[j] = r;
-    } else if (j < n_pad) {
-        PRec r;
-        r.x = r.y = r.z = kPadPos;
-        r.m32 = 0.0f;
-        r.pad = 0.0f;
-        p[j] = r;
-    }
-}
-
-__global__ __launch_bounds__(64) void k_pot_pass1(const PRec *__restrict__ p,
-                                                  int ntile, int i0, int ni,
-                                                  int n_iw, int nslice,
-                                                  double *__restrict__ part) {
-    const int ntask = n_iw * nslice;
-    const int per = (ntask + 7) >> 3;
-    const int task = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
-    if (task >= ntask) return;
-    const int s = task / n_iw;
-    const int iw = task - s * n_iw;
-    const int q = iw * 64 + threadIdx.x;
-    const bool act = q < ni;
-    const int tb = (int)(((long long)ntile * s) / nslice);
-    const int te = (int)(((long long)ntile * (s + 1)) / nslice);
-    double x0 = 0.0, y0 = 0.0, z0 = 0.0;
-    if (act) {
-        const PRec r = p[i0 + q];
-        x0 = r.x;
-        y0 = r.y;
-        z0 = r.z;
-    }
-    float a = 0.f;
-    double A = 0.0;
-    // Groups of four records; the next group is loaded while the current one
-    // is evaluated (the record array carries a spare tile past its end, so
-    // the last look-ahead stays in bounds).  Terms are added in j order.
-    constexpr int GP = 4;
-    PRec Jn[GP];
-#pragma unroll
-    for (int k = 0; k < GP; ++k) Jn[k] = p[tb * kTile + k];
-    for (int t = tb; t < te; ++t) {
-        const int jt = t * kTile;
-        for (int jg = 0; jg < kTile; jg += GP) {
-            PRec J[GP];
-#pragma unroll
-            for (int k = 0; k < GP; ++k) J[k] = Jn[k];
-#pragma unroll
-            for (int k = 0; k < GP; ++k) Jn[k] = p[jt + jg + GP + k];
-#pragma unroll
-            for (int k = 0; k < GP; ++k) {
-                const float fx = (float)(J[k].x - x0);
-                const float fy = (float)(J[k].y - y0);
-                const float fz = (float)(J[k].z - z0);
-                const float r2 = fmaf(fz, fz, fmaf(fy, fy, fx * fx));
-                const float term = J[k].m32 * __builtin_amdgcn_rsqf(r2);
-                a += (r2 > 0.0f) ? term : 0.0f;
-            }
-        }
-        A += (double)a;
-        a = 0.f;
-    }
-    if (act) part[(size_t)q * nslice + s] = A;
-}
-
-__global__ __launch_bounds__(256) void k_pot_pass2(const double *__restrict__ part,
-                                                   int ni, int nslice,
-                                                   double *__restrict__ pot) {
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= ni) return;
-    double s = 0.0;
-    for (int k = 0; k < nslice; ++k) s += part[(size_t)q * nslice + k];
-    pot[q] = s;
-}
-
-// ---------------------------------------------------------------------------
 // Launchers
 // ---------------------------------------------------------------------------
 
@@ -1591,26 +1495,6 @@ int pass2_ipb(int ni) {
     return ni >= 65536 ? kP2I : ni >= 32768 ? 16 : ni >= 16384 ? 8 : 4;
 }
 
-void launch_pack_p(hipStream_t st, const double *m, const double *x, int n,
-                   int n_pad, PRec *p, unsigned *err) {
-    if (n_pad <= 0) return;
-    hipLaunchKernelGGL(k_pack_p, dim3(cdiv(n_pad, 256)), dim3(256), 0, st, m, x,
-                       n, n_pad, p, err);
-}
-
-void launch_pot(hipStream_t st, const PRec *p, int n, int ntile, int i0,
-                int ni, int nslice, double *part, double *pot) {
-    (void)n;
-    if (ni <= 0) return;
-    const int n_iw = cdiv(ni, 64);
-    const int ntask = n_iw * nslice;
-    const int nblk = 8 * ((ntask + 7) / 8);
-    hipLaunchKernelGGL(k_pot_pass1, dim3(nblk), dim3(64), 0, st, p, ntile, i0,
-                       ni, n_iw, nslice, part);
-    hipLaunchKernelGGL(k_pot_pass2, dim3(cdiv(ni, 256)), dim3(256), 0, st, part,
-                       ni, nslice, pot);
-}
-
 // Resident wavefronts of a kernel launched in blocks of `block` threads.
 static int resident_waves_of(const void *fn, int block = 64) {
     int dev = 0;
@@ -1638,7 +1522,5 @@ int regf_resident_waves(int m_flag, int group, int prec) {
     return m_flag ? resident_waves_of((const void *)k_regf_pass1<true, 4>, 64 * kP1W)
                   : resident_waves_of((const void *)k_regf_pass1<false, 4>, 64 * kP1W);
 }
-
-int pot_resident_waves() { return resident_waves_of((const void *)k_pot_pass1); }
 
 }  // namespace gpunb
