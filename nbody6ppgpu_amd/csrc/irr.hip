@@ -6,9 +6,12 @@
 // State in HBM: one 128-byte predictor record per particle (x0, v0, f = a/2,
 // fd = jerk/6, m, t0 in FP64) and a neighbour table of nmax rows of lmax ints
 // (count, then 0-based indices).  set_jp / set_list stage their data on the
-// host; the next firr_vec uploads the staged records and rows in one copy each
-// and scatters them with a kernel, so per-particle Fortran calls cost no
-// device round trip.
+// host and the next firr_vec scatters it with a kernel, so per-particle
+// Fortran calls cost no device round trip.  A batched call
+// (gpunb_irr_set_jp, gpunb_irr_set_lists) copies the caller's arrays as they
+// are into one pinned block; the scatter kernel forms the records and rows
+// from it, from a device copy whose upload starts in the batched call when
+// the block is large, else from the pinned block itself.
 //
 // k_irr_force: one wavefront per active particle.  Every lane predicts its
 // list members with the FP64 polynomial of xbpredall.f:18-26 (the same
@@ -21,8 +24,10 @@
 // an empty list.  The reference evaluates the pairs in FP32 on double-single
 // positions; FP64 costs little here (a few tens of pairs per particle).
 #include <hip/hip_runtime.h>
+#include <hip/hip_ext.h>
 
 #include <algorithm>
+#include <atomic>
 #include <climits>
 #include <cmath>
 #include <cstdio>
@@ -32,6 +37,8 @@
 #include <mutex>
 #include <stdexcept>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "gpunb.h"
@@ -77,6 +84,21 @@ constexpr int kWavesPerBlock = 4;
 // one crosses the host link.
 constexpr int kOutChunks = 4;
 constexpr int kChunkMin = 4 * 8192;
+// Calls of up to kDirectMax bodies write their results to the mapped pinned
+// buffers from the force kernel itself.
+constexpr int kDirectMax = 2048;
+// Pairs of a call from which members are read from records predicted once
+// (N = 131072, 7.3M pairs: 0.150 against 0.176 ms of kernels; 1.9M pairs:
+// 564 against 553 us a call, the extra launch costing what it saves).
+constexpr long long kPreMin = 3000000;
+// Batched calls of at least kBlockMin bodies are staged as blocks, at most
+// kMaxBlocks of them at a time; a block of at least kUploadMin bytes is
+// uploaded by the copy engine while the host goes on, a smaller one read from
+// the host by the scatter kernel (8192 bodies, a call: 193 us with the line at
+// 1 MiB, 181 at 512 KiB, 179 at 256 KiB and below).
+constexpr int kBlockMin = 64;
+constexpr size_t kMaxBlocks = 8;
+constexpr size_t kUploadMin = 256 << 10;
 
 // A particle predicted to the call's time: position, velocity, mass.
 struct alignas(64) PRec {
@@ -180,37 +202,65 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void k_irr_force(
             bestj = oj;
         }
     }
-    if (lane == 0) {
-        acc[3 * (size_t)q + 0] = a0;
-        acc[3 * (size_t)q + 1] = a1;
-        acc[3 * (size_t)q + 2] = a2;
-        jrk[3 * (size_t)q + 0] = j0;
-        jrk[3 * (size_t)q + 1] = j1;
-        jrk[3 * (size_t)q + 2] = j2;
-        nnbid[q] = bestj == INT_MAX ? 0 : bestj + 1;
+    // Every lane holds the sums: one store per vector.
+    if (lane < 3) {
+        acc[3 * (size_t)q + lane] = lane == 0 ? a0 : lane == 1 ? a1 : a2;
+        jrk[3 * (size_t)q + lane] = lane == 0 ? j0 : lane == 1 ? j1 : j2;
     }
+    if (lane == 0) nnbid[q] = bestj == INT_MAX ? 0 : bestj + 1;
 }
 
-// Staged predictor records -> their slots.
-__global__ void k_irr_scatter_jp(int n, const int *__restrict__ addr,
-                                 const IRec *__restrict__ src,
-                                 IRec *__restrict__ jp) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < n) jp[addr[k]] = src[k];
-}
+// Staged data -> its slots, and the active indices of the call to the device,
+// in one launch: workgroups [0, bj) take 256 records each, [bj, bj + bl) four
+// list rows each (one wavefront per row), the rest 256 indices each.
+//   records: arrays x, v, f, fd [n][3], m, t0 [n] one after another (soa) and
+//            the slots; the caller's arrays as they are.
+//   rows:    hdr[3r] = slot, hdr[3r+1] = offset of the row in flat,
+//            hdr[3r+2] = count; flat: 0-based members.
+struct StageArgs {
+    int nj, nr, ni;
+    unsigned bj, bl;
+    const double *soa;
+    const int *slot;
+    IRec *jp;
+    const int *hdr, *flat;
+    int *list;
+    int lstride;
+    const int *idx_src;
+    int *idx;
+};
 
-// Staged list rows: hdr[3r] = slot, hdr[3r+1] = offset of the row in flat,
-// hdr[3r+2] = count; one wavefront per row (entries already 0-based).
-__global__ void k_irr_scatter_lists(int nrows, const int *__restrict__ hdr,
-                                    const int *__restrict__ flat,
-                                    int *__restrict__ list, int lstride) {
-    const int lane = threadIdx.x & 63;
-    const int r = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    if (r >= nrows) return;
-    const int slot = hdr[3 * r], off = hdr[3 * r + 1], cnt = hdr[3 * r + 2];
-    int *row = list + (size_t)slot * lstride;
-    if (lane == 0) row[0] = cnt;
-    for (int k = lane; k < cnt; k += 64) row[1 + k] = flat[off + k];
+__global__ __launch_bounds__(256) void k_irr_stage(StageArgs s) {
+    const unsigned b = blockIdx.x;
+    if (b < s.bj) {
+        const int k = b * 256 + threadIdx.x;
+        if (k >= s.nj) return;
+        const size_t n = (size_t)s.nj;
+        IRec r;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            r.x[c] = s.soa[3 * (size_t)k + c];
+            r.v[c] = s.soa[3 * (n + k) + c];
+            r.f[c] = s.soa[3 * (2 * n + k) + c];
+            r.fd[c] = s.soa[3 * (3 * n + k) + c];
+        }
+        r.m = s.soa[12 * n + k];
+        r.t0 = s.soa[13 * n + k];
+        r.pad[0] = r.pad[1] = 0.0;
+        s.jp[s.slot[k]] = r;
+    } else if (b < s.bj + s.bl) {
+        const int lane = threadIdx.x & 63;
+        const int r = (int)(b - s.bj) * 4 + (int)(threadIdx.x >> 6);
+        if (r >= s.nr) return;
+        const int slot = s.hdr[3 * r], off = s.hdr[3 * r + 1],
+                  cnt = s.hdr[3 * r + 2];
+        int *row = s.list + (size_t)slot * s.lstride;
+        if (lane == 0) row[0] = cnt;
+        for (int k = lane; k < cnt; k += 64) row[1 + k] = s.flat[off + k];
+    } else {
+        const int q = (int)(b - s.bj - s.bl) * 256 + threadIdx.x;
+        if (q < s.ni) s.idx[q] = s.idx_src[q];
+    }
 }
 
 // Device -> mapped pinned host copy of three ranges of n16[b] 16-byte units,
@@ -270,9 +320,32 @@ struct HBuf {
     }
 };
 
+// The data of one batched call (or of the merged per-particle calls), pinned:
+// records as the arrays and slots of k_irr_stage, rows as its headers and
+// members.
+struct Block {
+    bool rows = false;
+    int n = 0;
+    size_t nflat = 0;
+    HBuf<char> h;
+    DBuf<char> d;
+    const char *src = nullptr;   // where the device reads it
+    size_t ints_at() const { return rows ? 0 : (size_t)n * 14 * sizeof(double); }
+    size_t bytes() const {
+        return ints_at() + (rows ? 3 * (size_t)n + nflat : (size_t)n) * sizeof(int);
+    }
+    double *soa() { return (double *)h.p; }
+    int *ints() { return (int *)(h.p + ints_at()); }
+    void release() {
+        h.release();
+        d.release();
+    }
+};
+
 struct State {
     bool open = false;
     int nmax = 0, lstride = 0;
+    int dev = 0;
     hipStream_t st = nullptr;
     DBuf<IRec> jp;
     DBuf<PRec> pj;                            // slots predicted to a call's t
@@ -282,10 +355,13 @@ struct State {
     std::vector<int> jp_addr, jp_slot;        // jp_slot[a] = staged index or -1
     std::vector<int> ls_hdr, ls_flat, ls_slot;
     std::vector<int> nnb;                     // host mirror of the counts
-    HBuf<IRec> h_rec;
-    HBuf<int> h_int;
-    DBuf<IRec> d_rec;
-    DBuf<int> d_int;
+    std::vector<int> seen;                    // slot marks of a batched call
+    int seen_mark = 0;
+    // Blocks staged, in call order (older than anything staged per particle),
+    // and blocks at rest, kept for the next calls.
+    std::vector<Block *> blocks, idle;
+    HBuf<int> h_idx;
+    DBuf<int> d_idx;
     // results of a call: acc[ni_pad][3], jerk[ni_pad][3] (d_out, h_out) and
     // the nearest neighbours[ni_pad] (d_nn, h_nn), ni_pad = ni rounded up to
     // 64, so every part of them starts on a 16-byte boundary
@@ -307,17 +383,22 @@ State I;
 // inside an OpenMP parallel loop (intgrt.F:200-205), so they must be safe to
 // call concurrently: each thread appends to its own buffer, and the next
 // firr_vec (called from one thread, with no staging running) merges all
-// buffers, keeping the last value staged for each particle.
+// buffers, keeping the last value staged for each particle.  Batched calls
+// stage blocks, under the lock; one that follows per-particle calls which no
+// firr_vec has merged yet goes the per-particle way, so blocks are always the
+// older data.
 struct Stage {
     std::vector<IRec> rec;
     std::vector<int> rec_addr;   // 0-based slot per record
     std::vector<int> hdr;        // (slot, offset in flat, count) per row
     std::vector<int> flat;       // members, 0-based
+    std::atomic<bool> used{false};
     void clear() {
         rec.clear();
         rec_addr.clear();
         hdr.clear();
         flat.clear();
+        used.store(false, std::memory_order_relaxed);
     }
 };
 std::mutex g_stage_mu;
@@ -347,6 +428,7 @@ void stage_jp(int a, const double *x, const double *v, const double *f,
     r.m = m;
     r.t0 = t0;
     Stage &st = my_stage();
+    st.used.store(true, std::memory_order_release);
     st.rec.push_back(r);
     st.rec_addr.push_back(a - 1);
 }
@@ -358,6 +440,7 @@ void stage_list(int a, int cnt, const int *nb) {
     for (int k = 0; k < cnt; ++k)
         IREQ(nb[k] >= 1 && nb[k] <= I.nmax, "list member out of range [1, nmax]");
     Stage &st = my_stage();
+    st.used.store(true, std::memory_order_release);
     st.hdr.push_back(a - 1);
     st.hdr.push_back((int)st.flat.size());
     st.hdr.push_back(cnt);
@@ -397,8 +480,241 @@ void merge_stages() {
 void clear_stages() {
     std::lock_guard<std::mutex> g(g_stage_mu);
     for (Stage *st : g_stages) st->clear();
+    for (Block *b : I.blocks) I.idle.push_back(b);
+    I.blocks.clear();
 }
 
+// Copies of more than kSplitMin bytes are split over four threads: one core
+// moves them at a fraction of the memory's rate, but starting the threads
+// takes about 30 us (8192 bodies, a call: 192 us unsplit, 239 split; 131072
+// bodies staged and evaluated: 10.3 ms with a record and row at a time through
+// the per-particle buffers, 1.7 ms so).
+constexpr size_t kSplitMin = 2 << 20;
+template <class F>
+void split(size_t n, size_t bytes, F f) {
+    constexpr int T = 4;
+    std::thread th[T - 1];
+    size_t done = 0;
+    int started = 0;
+    if (bytes >= kSplitMin) {
+        try {
+            for (; started < T - 1; ++started) {
+                const size_t lo = done, hi = n * (started + 1) / T;
+                th[started] = std::thread([=] { f(lo, hi); });
+                done = hi;
+            }
+        } catch (const std::system_error &) {
+            // No more threads: this one does the rest.
+        }
+    }
+    f(done, n);
+    for (int k = 0; k < started; ++k) th[k].join();
+}
+
+// A block that can hold what *want says, from the idle ones or new.
+Block *take_block(bool rows, int n, size_t nflat) {
+    Block *b = nullptr;
+    if (!I.idle.empty()) {
+        // The one whose buffer fits best: the smallest that is large enough,
+        // else the largest.
+        Block w;
+        w.rows = rows;
+        w.n = n;
+        w.nflat = nflat;
+        const size_t need = w.bytes();
+        size_t at = 0;
+        for (size_t k = 1; k < I.idle.size(); ++k) {
+            const size_t c = I.idle[k]->h.cap, a = I.idle[at]->h.cap;
+            if (a < need ? c > a : (c >= need && c < a)) at = k;
+        }
+        b = I.idle[at];
+        I.idle.erase(I.idle.begin() + at);
+    } else {
+        b = new Block;
+    }
+    b->rows = rows;
+    b->n = n;
+    b->nflat = nflat;
+    b->src = nullptr;
+    try {
+        b->h.ensure(b->bytes());
+    } catch (...) {
+        I.idle.push_back(b);
+        throw;
+    }
+    return b;
+}
+
+// Start the upload of a large block; small ones are read where they are.
+void place_block(Block *b) {
+    const size_t n = b->bytes();
+    if (n >= kUploadMin) {
+        int cur = 0;
+        ICHK(hipGetDevice(&cur));
+        if (cur != I.dev) ICHK(hipSetDevice(I.dev));
+        hipError_t rc = hipSuccess;
+        try {
+            b->d.ensure(n);
+            rc = hipMemcpyAsync(b->d.p, b->h.p, n, hipMemcpyHostToDevice, I.st);
+        } catch (...) {
+            if (cur != I.dev) (void)hipSetDevice(cur);
+            throw;
+        }
+        if (cur != I.dev) ICHK(hipSetDevice(cur));
+        ICHK(rc);
+        b->src = b->d.p;
+    } else {
+        void *p = nullptr;
+        ICHK(hipHostGetDevicePointer(&p, b->h.p, 0));
+        b->src = (const char *)p;
+    }
+}
+
+// Whether a batched call of n bodies is staged as a block (lock held).
+bool block_ok(int n) {
+    if (n < kBlockMin || I.blocks.size() >= kMaxBlocks) return false;
+    if (!I.jp_rec.empty() || !I.ls_hdr.empty()) return false;
+    for (Stage *st : g_stages)
+        if (st->used.load(std::memory_order_acquire)) return false;
+    return true;
+}
+
+// Addresses of a batched call in range (an error otherwise) and each listed
+// once (false otherwise: the per-particle way keeps the last).
+bool addresses_once(int n, const int *addr) {
+    bool ascending = true, range = true;
+    for (int q = 0; q < n; ++q) {
+        range = range && addr[q] >= 1 && addr[q] <= I.nmax;
+        ascending = ascending && (q == 0 || addr[q] > addr[q - 1]);
+    }
+    IREQ(range, "address out of range [1, nmax]");
+    if (ascending) return true;
+    if (++I.seen_mark == INT_MAX) {
+        std::fill(I.seen.begin(), I.seen.end(), 0);
+        I.seen_mark = 1;
+    }
+    for (int q = 0; q < n; ++q) {
+        int &m = I.seen[addr[q] - 1];
+        if (m == I.seen_mark) return false;
+        m = I.seen_mark;
+    }
+    return true;
+}
+
+bool block_jp(int n, const int *addr, const double *x, const double *v,
+              const double *f, const double *fd, const double *m,
+              const double *t0) {
+    std::lock_guard<std::mutex> g(g_stage_mu);
+    if (!block_ok(n) || !addresses_once(n, addr)) return false;
+    Block *b = take_block(false, n, 0);
+    I.blocks.push_back(b);
+    try {
+        double *h = b->soa();
+        int *slot = b->ints();
+        const size_t N = (size_t)n;
+        split(N, b->bytes(), [=](size_t lo, size_t hi) {
+            const double *v3[4] = {x, v, f, fd};
+            for (int c = 0; c < 4; ++c)
+                memcpy(h + 3 * (c * N + lo), v3[c] + 3 * lo,
+                       3 * (hi - lo) * sizeof(double));
+            memcpy(h + 12 * N + lo, m + lo, (hi - lo) * sizeof(double));
+            memcpy(h + 13 * N + lo, t0 + lo, (hi - lo) * sizeof(double));
+            for (size_t q = lo; q < hi; ++q) slot[q] = addr[q] - 1;
+        });
+        place_block(b);
+    } catch (...) {
+        I.blocks.pop_back();
+        I.idle.push_back(b);
+        throw;
+    }
+    return true;
+}
+
+bool block_lists(int n, const int *addr, const int *nnb, const int *members) {
+    std::lock_guard<std::mutex> g(g_stage_mu);
+    if (!block_ok(n)) return false;
+    size_t nf = 0;
+    for (int q = 0; q < n; ++q) {
+        IREQ(nnb[q] >= 0 && nnb[q] <= I.lstride - 1, "list longer than lmax - 1");
+        nf += (size_t)nnb[q];
+    }
+    if (nf > (size_t)INT_MAX || !addresses_once(n, addr)) return false;
+    Block *b = take_block(true, n, nf);
+    I.blocks.push_back(b);
+    try {
+        int *hdr = b->ints(), *flat = hdr + 3 * (size_t)n;
+        int off = 0;
+        for (int q = 0; q < n; ++q) {
+            hdr[3 * (size_t)q] = addr[q] - 1;
+            hdr[3 * (size_t)q + 1] = off;
+            hdr[3 * (size_t)q + 2] = nnb[q];
+            off += nnb[q];
+        }
+        std::atomic<bool> bad{false};
+        std::atomic<bool> *pbad = &bad;
+        const unsigned nmax = (unsigned)I.nmax;
+        split(nf, nf * sizeof(int), [=](size_t lo, size_t hi) {
+            unsigned out = 0;
+            for (size_t k = lo; k < hi; ++k) {
+                const int j = members[k] - 1;
+                out |= (unsigned)j >= nmax;
+                flat[k] = j;
+            }
+            if (out) pbad->store(true, std::memory_order_relaxed);
+        });
+        IREQ(!bad.load(), "list member out of range [1, nmax]");
+        place_block(b);
+        for (int q = 0; q < n; ++q) I.nnb[addr[q] - 1] = nnb[q];
+    } catch (...) {
+        I.blocks.pop_back();
+        I.idle.push_back(b);
+        throw;
+    }
+    return true;
+}
+
+// What the per-particle calls staged, as blocks.
+void block_merged() {
+    const size_t nj = I.jp_rec.size();
+    if (nj) {
+        Block *b = take_block(false, (int)nj, 0);
+        I.blocks.push_back(b);
+        double *h = b->soa();
+        for (size_t k = 0; k < nj; ++k) {
+            const IRec &r = I.jp_rec[k];
+            for (int c = 0; c < 3; ++c) {
+                h[3 * k + c] = r.x[c];
+                h[3 * (nj + k) + c] = r.v[c];
+                h[3 * (2 * nj + k) + c] = r.f[c];
+                h[3 * (3 * nj + k) + c] = r.fd[c];
+            }
+            h[12 * nj + k] = r.m;
+            h[13 * nj + k] = r.t0;
+        }
+        memcpy(b->ints(), I.jp_addr.data(), nj * sizeof(int));
+        place_block(b);
+        for (int s : I.jp_addr) I.jp_slot[s] = -1;
+        I.jp_rec.clear();
+        I.jp_addr.clear();
+    }
+    size_t nr = 0;
+    for (size_t r = 0; r < I.ls_hdr.size(); r += 3) nr += I.ls_hdr[r] >= 0;
+    if (nr) {
+        Block *b = take_block(true, (int)nr, I.ls_flat.size());
+        I.blocks.push_back(b);
+        int *hdr = b->ints();
+        for (size_t r = 0; r < I.ls_hdr.size(); r += 3)
+            if (I.ls_hdr[r] >= 0) {
+                memcpy(hdr, I.ls_hdr.data() + r, 3 * sizeof(int));
+                hdr += 3;
+                I.ls_slot[I.ls_hdr[r]] = -1;
+            }
+        memcpy(hdr, I.ls_flat.data(), I.ls_flat.size() * sizeof(int));
+        place_block(b);
+    }
+    I.ls_hdr.clear();
+    I.ls_flat.clear();
+}
 
 double wtime() {
     struct timespec ts;
@@ -424,6 +740,7 @@ void do_open(int nmax, int lmax, int rank) {
     for (int c = 0; c < kOutChunks; ++c)
         ICHK(hipEventCreateWithFlags(&I.part[c], hipEventDisableTiming));
     I.last_kernel_ms = 0.0;
+    ICHK(hipGetDevice(&I.dev));
     I.nmax = nmax;
     I.lstride = lmax;
     I.jp.ensure((size_t)nmax);
@@ -435,6 +752,8 @@ void do_open(int nmax, int lmax, int rank) {
     I.jp_slot.assign(nmax, -1);
     I.ls_slot.assign(nmax, -1);
     I.nnb.assign(nmax, 0);
+    I.seen.assign(nmax, 0);
+    I.seen_mark = 0;
     I.jp_rec.clear();
     I.jp_addr.clear();
     I.ls_hdr.clear();
@@ -457,12 +776,16 @@ void do_close(int rank) {
     I.jp.release();
     I.pj.release();
     I.list.release();
-    I.d_rec.release();
-    I.d_int.release();
+    I.d_idx.release();
     I.d_out.release();
     I.d_nn.release();
-    I.h_rec.release();
-    I.h_int.release();
+    I.h_idx.release();
+    clear_stages();
+    for (Block *b : I.idle) {
+        b->release();
+        delete b;
+    }
+    I.idle.clear();
     I.h_out.release();
     I.h_nn.release();
     (void)hipEventDestroy(I.ev0);
@@ -478,98 +801,96 @@ void do_close(int rank) {
     if (!quiet()) fprintf(stderr, "Closing irr_simd lib. MI355X ver. - rank: %d\n", rank);
 }
 
-// Upload the staged records and list rows, scatter them, then (ni > 0) the
-// force of addr[] at t; the host waits only for each part of the results
-// (one part below kChunkMin bodies).  Layout of the pinned int buffer:
-// [jp slots (nj)] [row headers (3 nr)] [members] [i (ni)].
+// Scatter the staged blocks, then (ni > 0) the force of addr[] at t; the host
+// waits only for each part of the results (one part below kChunkMin bodies).
 void flush_and_force(double t, int ni, const int *addr, double *acc,
                      double *jrk, int *nnbid) {
+    I.h_idx.ensure((size_t)ni);
+    I.d_idx.ensure((size_t)ni);
     merge_stages();
-    const size_t nj = I.jp_rec.size();
-    std::vector<int> hdr;
-    hdr.reserve(I.ls_hdr.size());
-    for (size_t r = 0; r < I.ls_hdr.size(); r += 3)
-        if (I.ls_hdr[r] >= 0)
-            hdr.insert(hdr.end(), I.ls_hdr.begin() + r, I.ls_hdr.begin() + r + 3);
-    const size_t nr = hdr.size() / 3, nf = I.ls_flat.size();
-    const size_t o_hdr = nj, o_flat = o_hdr + 3 * nr, o_idx = o_flat + nf;
-    const size_t nint = o_idx + (size_t)ni;
     long long pairs = 0;
-    if (nint) {
-        I.h_int.ensure(nint);
-        I.d_int.ensure(nint);
-        int *h = I.h_int.p;
-        memcpy(h, I.jp_addr.data(), nj * sizeof(int));
-        memcpy(h + o_hdr, hdr.data(), 3 * nr * sizeof(int));
-        memcpy(h + o_flat, I.ls_flat.data(), nf * sizeof(int));
-        for (int q = 0; q < ni; ++q) {
-            const int a = addr[q];
-            IREQ(a >= 1 && a <= I.nmax, "address out of range [1, nmax]");
-            h[o_idx + q] = a - 1;
+    for (int q = 0; q < ni; ++q) {
+        const int a = addr[q];
+        IREQ(a >= 1 && a <= I.nmax, "address out of range [1, nmax]");
+        I.h_idx.p[q] = a - 1;
+        pairs += I.nnb[a - 1];
+    }
+    block_merged();
+    // One launch per pair of a record and a row block, in staging order (a
+    // later block overwrites an earlier one's slots); the last one also
+    // brings the call's indices.
+    StageArgs s = {};
+    s.jp = I.jp.p;
+    s.list = I.list.p;
+    s.lstride = I.lstride;
+    auto launch = [&] {
+        s.bj = (unsigned)((s.nj + 255) / 256);
+        s.bl = (unsigned)((s.nr + 3) / 4);
+        const unsigned nb = s.bj + s.bl + (unsigned)((s.ni + 255) / 256);
+        if (nb) hipLaunchKernelGGL(k_irr_stage, dim3(nb), dim3(256), 0, I.st, s);
+        s.nj = s.nr = 0;
+    };
+    for (Block *b : I.blocks) {
+        if (b->rows ? s.nr : s.nj) launch();
+        if (b->rows) {
+            s.nr = b->n;
+            s.hdr = (const int *)b->src;
+            s.flat = s.hdr + 3 * (size_t)b->n;
+        } else {
+            s.nj = b->n;
+            s.soa = (const double *)b->src;
+            s.slot = (const int *)(b->src + b->ints_at());
         }
-        ICHK(hipMemcpyAsync(I.d_int.p, h, nint * sizeof(int),
-                            hipMemcpyHostToDevice, I.st));
     }
-    if (nj) {
-        I.h_rec.ensure(nj);
-        I.d_rec.ensure(nj);
-        memcpy(I.h_rec.p, I.jp_rec.data(), nj * sizeof(IRec));
-        ICHK(hipMemcpyAsync(I.d_rec.p, I.h_rec.p, nj * sizeof(IRec),
-                            hipMemcpyHostToDevice, I.st));
-        hipLaunchKernelGGL(k_irr_scatter_jp, dim3((unsigned)((nj + 255) / 256)),
-                           dim3(256), 0, I.st, (int)nj, I.d_int.p, I.d_rec.p,
-                           I.jp.p);
+    if (ni > 0) {
+        void *hi = nullptr;
+        ICHK(hipHostGetDevicePointer(&hi, I.h_idx.p, 0));
+        s.ni = ni;
+        s.idx_src = (const int *)hi;
+        s.idx = I.d_idx.p;
     }
-    if (nr)
-        hipLaunchKernelGGL(k_irr_scatter_lists, dim3((unsigned)((nr + 3) / 4)),
-                           dim3(256), 0, I.st, (int)nr, I.d_int.p + o_hdr,
-                           I.d_int.p + o_flat, I.list.p, I.lstride);
-    for (int s : I.jp_addr) I.jp_slot[s] = -1;
-    for (size_t r = 0; r < I.ls_hdr.size(); r += 3)
-        if (I.ls_hdr[r] >= 0) I.ls_slot[I.ls_hdr[r]] = -1;
-    // Counts of the members sent now are already in the host mirror.
-    for (int q = 0; q < ni; ++q) pairs += I.nnb[addr[q] - 1];
-    I.jp_rec.clear();
-    I.jp_addr.clear();
-    I.ls_hdr.clear();
-    I.ls_flat.clear();
+    launch();
     if (ni > 0) {
         const size_t np = ((size_t)ni + 63) & ~(size_t)63;
         I.d_out.ensure(np * 6);
         I.d_nn.ensure(np);
         I.h_out.ensure(np * 6);
         I.h_nn.ensure(np);
-        ICHK(hipEventRecord(I.ev0, I.st));
-        // Predict every slot once when the call's pairs outnumber the slots
-        // threefold: each member then costs a 64-byte read instead of a
-        // 128-byte read and its prediction.
-        const bool pre = pairs > 3LL * I.nmax;
+        void *ho = nullptr, *hn = nullptr;
+        ICHK(hipHostGetDevicePointer(&ho, I.h_out.p, 0));
+        ICHK(hipHostGetDevicePointer(&hn, I.h_nn.p, 0));
+        const bool direct = ni <= kDirectMax;
+        double *out = direct ? (double *)ho : I.d_out.p;
+        int *nn = direct ? (int *)hn : I.d_nn.p;
+        // Predict every slot once when the call's pairs are many and outnumber
+        // the slots threefold: each member then costs a 64-byte read instead of a
+        // 128-byte read and its prediction.  The events of the kernel timing
+        // are those of the launches themselves (separate records would each
+        // hold up the stream).
+        const bool pre = pairs > 3LL * I.nmax && pairs > kPreMin;
         if (pre) {
             I.pj.ensure((size_t)I.nmax);
-            hipLaunchKernelGGL(k_irr_predict, dim3((unsigned)((I.nmax + 255) / 256)),
-                               dim3(256), 0, I.st, I.nmax, t, I.jp.p, I.pj.p);
+            hipExtLaunchKernelGGL(k_irr_predict, dim3((unsigned)((I.nmax + 255) / 256)),
+                                  dim3(256), 0, I.st, I.ev0, nullptr, 0, I.nmax,
+                                  t, I.jp.p, I.pj.p);
         }
         const dim3 grid((unsigned)((ni + kWavesPerBlock - 1) / kWavesPerBlock));
         if (pre)
-            hipLaunchKernelGGL(k_irr_force<true>, grid, dim3(64 * kWavesPerBlock),
-                               0, I.st, ni, I.d_int.p + o_idx, t, I.jp.p,
-                               I.pj.p, I.list.p, I.lstride, I.d_out.p,
-                               I.d_out.p + 3 * np, I.d_nn.p);
+            hipExtLaunchKernelGGL(k_irr_force<true>, grid, dim3(64 * kWavesPerBlock),
+                                  0, I.st, nullptr, I.ev1, 0, ni, I.d_idx.p, t,
+                                  I.jp.p, I.pj.p, I.list.p, I.lstride, out,
+                                  out + 3 * np, nn);
         else
-            hipLaunchKernelGGL(k_irr_force<false>, grid, dim3(64 * kWavesPerBlock),
-                               0, I.st, ni, I.d_int.p + o_idx, t, I.jp.p,
-                               (const PRec *)nullptr, I.list.p, I.lstride,
-                               I.d_out.p, I.d_out.p + 3 * np, I.d_nn.p);
-        ICHK(hipEventRecord(I.ev1, I.st));
+            hipExtLaunchKernelGGL(k_irr_force<false>, grid, dim3(64 * kWavesPerBlock),
+                                  0, I.st, I.ev0, I.ev1, 0, ni, I.d_idx.p, t,
+                                  I.jp.p, (const PRec *)nullptr, I.list.p,
+                                  I.lstride, out, out + 3 * np, nn);
         // Part c: bodies q0 .. q0 + nq (q0 a multiple of 64), copied by one
         // launch to the mapped h_out / h_nn; a byte count is rounded up to
         // 16, which stays inside the padded arrays.
         const int nchunk = ni >= kChunkMin ? kOutChunks : 1;
         const int per = (int)((((size_t)ni + nchunk - 1) / nchunk + 63) & ~(size_t)63);
-        void *ho = nullptr, *hn = nullptr;
-        ICHK(hipHostGetDevicePointer(&ho, I.h_out.p, 0));
-        ICHK(hipHostGetDevicePointer(&hn, I.h_nn.p, 0));
-        for (int c = 0; c < nchunk; ++c) {
+        for (int c = 0; c < nchunk && !direct; ++c) {
             const size_t q0 = (size_t)c * per;
             if (q0 >= (size_t)ni) break;
             const size_t nq = std::min<size_t>(ni - q0, per);
@@ -593,7 +914,10 @@ void flush_and_force(double t, int ni, const int *addr, double *acc,
             const size_t q0 = (size_t)c * per;
             if (q0 >= (size_t)ni) break;
             const size_t nq = std::min<size_t>(ni - q0, per);
-            ICHK(hipEventSynchronize(I.part[c]));
+            if (direct)
+                ICHK(hipStreamSynchronize(I.st));
+            else
+                ICHK(hipEventSynchronize(I.part[c]));
             memcpy(acc + 3 * q0, I.h_out.p + 3 * q0, 3 * nq * sizeof(double));
             memcpy(jrk + 3 * q0, I.h_out.p + 3 * (np + q0), 3 * nq * sizeof(double));
             if (nnbid) memcpy(nnbid + q0, I.h_nn.p + q0, nq * sizeof(int));
@@ -606,8 +930,16 @@ void flush_and_force(double t, int ni, const int *addr, double *acc,
         I.ninter += pairs;
     } else {
         ICHK(hipGetLastError());
-        // The pinned staging buffers are reused by the next call.
-        if (nint || nj) ICHK(hipStreamSynchronize(I.st));
+        // The pinned blocks are reused by the next calls.
+        if (!I.blocks.empty()) ICHK(hipStreamSynchronize(I.st));
+    }
+    std::lock_guard<std::mutex> g(g_stage_mu);
+    for (Block *b : I.blocks) I.idle.push_back(b);
+    I.blocks.clear();
+    while (I.idle.size() > kMaxBlocks) {
+        I.idle.back()->release();
+        delete I.idle.back();
+        I.idle.pop_back();
     }
 }
 
@@ -682,6 +1014,7 @@ IRR_EXPORT int gpunb_irr_set_jp(int n, const int *addr, const double *x,
                                 const double *t0) {
     return gpunb::run_guarded("gpunb_irr_set_jp", [&] {
         IREQ(I.open, "irr_simd is not open");
+        if (block_jp(n, addr, x, v, f, fd, m, t0)) return;
         for (int q = 0; q < n; ++q)
             stage_jp(addr[q], x + 3 * (size_t)q, v + 3 * (size_t)q,
                      f + 3 * (size_t)q, fd + 3 * (size_t)q, m[q], t0[q]);
@@ -694,6 +1027,7 @@ IRR_EXPORT int gpunb_irr_set_lists(int n, const int *addr, const int *nnb,
                                    const int *members) {
     return gpunb::run_guarded("gpunb_irr_set_lists", [&] {
         IREQ(I.open, "irr_simd is not open");
+        if (block_lists(n, addr, nnb, members)) return;
         size_t off = 0;
         for (int q = 0; q < n; ++q) {
             stage_list(addr[q], nnb[q], members + off);
