@@ -953,8 +953,8 @@ void do_regf(int ni, const double *h2, const double *dtr, const double (*xi)[3],
     est = std::min(est, list_cap);
     const size_t first = round_up16(off_l + (size_t)est * sizeof(int));
     S.h_res.ensure(first);
-    launch_copy_to_host(S.st, S.d_res.p, host_dev_ptr(S.h_res.p), first, S.err.p,
-                        (unsigned *)host_dev_ptr(S.h_err.p));
+    launch_copy_to_host(S.st, S.d_res.p, host_dev_ptr(S.h_res.p), first, off_l,
+                        d_total, S.err.p, (unsigned *)host_dev_ptr(S.h_err.p));
     HIPCHK(hipStreamSynchronize(S.st));
     err_check();
     double t1 = wtime();

@@ -279,10 +279,12 @@ int pass2_ipb(int ni);   // pass-2 i per workgroup for a launch of ni
 int pass2_sortcap(int nnbmax);
 constexpr int kMaxNnbmax = 4000;
 void launch_zero_int(hipStream_t st, int *p, int n);
-// bytes (a multiple of 16, both pointers 16-byte aligned) from device memory
-// to a mapped pinned host buffer, and *err to *herr (host-mapped).
+// At most bytes (a multiple of 16, both pointers 16-byte aligned) from device
+// memory to a mapped pinned host buffer: the first `fixed`, and *nlast ints
+// after them; and *err to *herr (host-mapped).
 void launch_copy_to_host(hipStream_t st, const void *src, void *dst,
-                         size_t bytes, const unsigned *err, unsigned *herr);
+                         size_t bytes, size_t fixed, const int *nlast,
+                         const unsigned *err, unsigned *herr);
 // bytes (a multiple of 16, both pointers 16-byte aligned) from a mapped
 // pinned host buffer to device memory, and *zero = 0.
 void launch_copy_from_host(hipStream_t st, const void *src, void *dst,

@@ -279,9 +279,14 @@ __global__ __launch_bounds__(256) void k_jget(int n, const JRec *__restrict__ jp
 // wavefront writes whole 1 KiB runs across the host link), plus the error
 // word: the results of a host-array call come back without a copy-engine
 // transfer, in stream order.
+// The last *nlast ints of them are as long as the call found out: from byte
+// `fixed` on only those are copied.
 __global__ __launch_bounds__(256) void k_copy_to_host(
     const uint4 *__restrict__ src, uint4 *__restrict__ dst, size_t n16,
+    size_t fixed, const int *__restrict__ nlast,
     const unsigned *__restrict__ err, unsigned *__restrict__ herr) {
+    const size_t need = (fixed + (size_t)*nlast * sizeof(int) + 15) / 16;
+    if (need < n16) n16 = need;
     const size_t stride = (size_t)gridDim.x * blockDim.x;
     for (size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x; k < n16;
          k += stride)
@@ -1098,8 +1103,9 @@ __global__ __launch_bounds__(64 * kP1W, p1_waves(G)) void k_regf_pass1_f64_q(
 // memory round trips in all, not for a few per i.  A list of up to 64 is one
 // entry per lane, placed by its rank among the others (16-byte broadcast
 // reads of the LDS row).  A longer one is ranked in chunks of 64 and its
-// entries placed by binary search in the other chunks: n^2 / 64 compares per
-// lane would make the longest lists the launch's end.
+// entries placed by binary search in the other chunks, by its wavefront or,
+// above kP2Own entries, by the whole workgroup: n^2 / 64 compares per lane, or
+// one wavefront for the longest lists, would make them the launch's end.
 //
 // Bound: latency (a wavefront's chain of dependent loads).  Before, an i at a
 // time with lanes over the slices, every entry ranked against all others:
@@ -1116,14 +1122,35 @@ __global__ __launch_bounds__(64 * kP1W, p1_waves(G)) void k_regf_pass1_f64_q(
 constexpr int kP2I = 32;
 constexpr int kP2W = kP2I / 4;   // i per wavefront, at most
 constexpr int kP2U = 8;          // slice partials loaded together
+constexpr int kP2Own = 256;      // entries of a list one wavefront sorts
+static_assert(kP2Own <= 64 * kP2W, "its LDS part (pass2_sortcap)");
 
-// Entries of the ascending LDS run a[0, m) (m <= 64) below v.
-__device__ inline int run_below(const int *a, int m, int v) {
-    int pos = 0;
+// Entries below v of the ascending LDS runs of 64 (the last one of n - 64
+// (nc - 1)) of rows, run `own` left out.  Four runs at a time: the binary
+// searches are chains of dependent LDS reads.
+__device__ inline int runs_below(const int *rows, int n, int nc, int own, int v) {
+    int sum = 0;
+    for (int d0 = 0; d0 < nc; d0 += 4) {
+        int pos[4], m[4];
 #pragma unroll
-    for (int s = 32; s >= 1; s >>= 1)
-        if (pos + s <= m && a[pos + s - 1] < v) pos += s;
-    return pos + ((pos < m && a[pos] < v) ? 1 : 0);
+        for (int u = 0; u < 4; ++u) {
+            const int d = d0 + u;
+            pos[u] = 0;
+            m[u] = d < nc && d != own ? min(64, n - 64 * d) : 0;
+        }
+#pragma unroll
+        for (int s = 32; s >= 1; s >>= 1)
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (pos[u] + s <= m[u] &&
+                    rows[64 * (d0 + u) + pos[u] + s - 1] < v)
+                    pos[u] += s;
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (pos[u] < m[u] && rows[64 * (d0 + u) + pos[u]] < v) ++pos[u];
+        sum += (pos[0] + pos[1]) + (pos[2] + pos[3]);
+    }
+    return sum;
 }
 
 // Entries below v among the first n of an LDS row (n rounded up to 4 reads
@@ -1131,6 +1158,7 @@ __device__ inline int run_below(const int *a, int m, int v) {
 __device__ inline int row_below(const int *row, int n, int v) {
     const int4 *r4 = reinterpret_cast<const int4 *>(row);
     int below = 0;
+#pragma unroll 4
     for (int k = 0; 4 * k < n; ++k) {
         const int4 w = r4[k];
         below += (w.x < v) + (w.y < v) + (w.z < v) + (w.w < v);
@@ -1138,20 +1166,20 @@ __device__ inline int row_below(const int *row, int n, int v) {
     return below;
 }
 
-// The lane's (r2, j) minimum over the wavefront, r2 first: the winning j (-1
-// if every r2 is infinite).
-__device__ inline int wave_nearest(double r2, int j) {
+// The (r2, j) minimum over the lanes of the wavefront, r2 first, in every
+// lane (j INT_MAX if every r2 is infinite).
+__device__ inline void wave_nearest(double &r2, int &j) {
     double m = r2;
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) m = fmin(m, __shfl_xor(m, o));
-    if (!(m < INFINITY)) return -1;
-    unsigned long long at = __ballot(r2 == m);
+    unsigned long long at = m < INFINITY ? __ballot(r2 == m) : 0ull;
     int best = INT_MAX;
     while (at) {
         best = min(best, __builtin_amdgcn_readlane(j, __builtin_ctzll(at)));
         at &= at - 1;
     }
-    return best;
+    r2 = m;
+    j = best;
 }
 
 template <bool NN>
@@ -1168,6 +1196,8 @@ __global__ __launch_bounds__(256) void k_regf_pass2(
     unsigned *__restrict__ err) {
     __shared__ int s_tot[kP2I];
     __shared__ int s_off[kP2I];
+    __shared__ double s_br2[4];
+    __shared__ int s_bj[4];
     extern __shared__ __align__(16) int s_rows[];   // [4][sortcap]
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1286,61 +1316,114 @@ __global__ __launch_bounds__(256) void k_regf_pass2(
                 r2 = sq3d(J.x - xi[q], J.y - xi[q + 1], J.z - xi[q + 2]);
                 if (!(r2 > 0.0)) r2 = INFINITY;
             }
-            const int b = wave_nearest(r2, jj[r]);
-            if (lane == r) best = b;
+            int b = jj[r];
+            wave_nearest(r2, b);
+            if (lane == r && b != INT_MAX) best = b;
         }
     }
 
-    // Longer lists, one at a time over the wavefront's whole LDS part.
+    // Longer lists of [b, b + n) of list i, by the threads t of nt (one
+    // wavefront, or the workgroup: sync holds them together) over lds; the
+    // nearest neighbour's (r2, j) per wavefront in br2, bj.
+    double br2 = INFINITY;
+    int bj = INT_MAX;
+    auto longer = [&](int i, int n, int o, int *__restrict__ lds, int t, int nt,
+                      auto sync) {
+        const int *__restrict__ e = nbl + (size_t)i * cap;
+        const size_t q = 3 * (size_t)i;
+        const int nc = (n + 63) >> 6;
+        br2 = INFINITY;
+        bj = INT_MAX;
+        sync();
+        // Four entries per thread at a time: their loads, and the gathers
+        // that follow them, are in flight together.
+        for (int k0 = t; k0 < 64 * nc; k0 += 4 * nt) {
+            int p[4], j[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int k = k0 + u * nt;
+                p[u] = k < n ? e[k] : -1;
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                j[u] = p[u] < 0 ? INT_MAX : jidx ? jidx[p[u]] : p[u];
+            if (NN) {
+                double r2[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    r2[u] = INFINITY;
+                    if (p[u] >= 0) {
+                        const JRec &J = jps[p[u]];
+                        r2[u] = sq3d(J.x - xi[q], J.y - xi[q + 1], J.z - xi[q + 2]);
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    if (r2[u] > 0.0 &&
+                        (r2[u] < br2 || (r2[u] == br2 && j[u] < bj))) {
+                        br2 = r2[u];
+                        bj = j[u];
+                    }
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int k = k0 + u * nt;
+                if (k < 64 * nc) lds[k] = j[u];
+            }
+        }
+        if (NN) wave_nearest(br2, bj);
+        sync();
+        // Every chunk in ascending order, a wavefront per chunk (its LDS
+        // accesses are in order: a chunk is read whole before it is
+        // rewritten).
+        const int c0 = __builtin_amdgcn_readfirstlane(t >> 6), dc = nt >> 6;
+        for (int c = c0; c < nc; c += dc) {
+            const int v = lds[64 * c + lane];
+            const int m = min(64, n - 64 * c);
+            const int below = row_below(lds + 64 * c, m, v);
+            __threadfence_block();
+            if (lane < m) lds[64 * c + below] = v;
+        }
+        sync();
+        for (int c = c0; c < nc; c += dc) {
+            const int v = lds[64 * c + lane];
+            const int below = lane + runs_below(lds, n, nc, c, v);
+            if (64 * c + lane < n) list[o + below] = v;
+        }
+    };
     for (int r = 0; r < niw; ++r) {
         const int n = __builtin_amdgcn_readlane(tot, r);
         const int o = __builtin_amdgcn_readlane(off, r);
-        if (o < 0 || n <= 64) continue;
-        const int *__restrict__ e = nbl + (size_t)(ib + r) * cap;
-        const size_t q = 3 * (size_t)(ib + r);
-        double br2 = INFINITY;
-        int bj = INT_MAX;
-        __threadfence_block();
-        const int nc = (n + 63) >> 6;
-        for (int k = lane; k < 64 * nc; k += 64) {
-            int j = INT_MAX;
-            if (k < n) {
-                const int p = e[k];
-                j = jidx ? jidx[p] : p;
-                if (NN) {
-                    const JRec &J = jps[p];
-                    const double r2 =
-                        sq3d(J.x - xi[q], J.y - xi[q + 1], J.z - xi[q + 2]);
-                    if (r2 > 0.0 && (r2 < br2 || (r2 == br2 && j < bj))) {
-                        br2 = r2;
-                        bj = j;
-                    }
-                }
-            }
-            rows[k] = j;
-        }
-        __threadfence_block();
-        // Every chunk in ascending order (the wavefront's LDS accesses are
-        // in order: a chunk is read whole before it is rewritten).
-        for (int c = 0; c < nc; ++c) {
-            const int v = rows[64 * c + lane];
-            const int m = min(64, n - 64 * c);
-            const int below = row_below(rows + 64 * c, m, v);
-            __threadfence_block();
-            if (lane < m) rows[64 * c + below] = v;
-        }
-        __threadfence_block();
-        for (int c = 0; c < nc; ++c) {
-            const int v = rows[64 * c + lane];
-            int below = lane;
-            for (int d = 0; d < nc; ++d)
-                if (d != c)
-                    below += run_below(rows + 64 * d, min(64, n - 64 * d), v);
-            if (64 * c + lane < n) list[o + below] = v;
-        }
+        if (o < 0 || n <= 64 || n > kP2Own) continue;
+        longer(ib + r, n, o, rows, lane, 64, [] { __threadfence_block(); });
+        if (NN && lane == r && bj != INT_MAX) best = bj;
+    }
+    const int tl = lane < ipb ? s_tot[lane] : 0;
+    const int ol = lane < ipb ? s_off[lane] : -1;
+    unsigned long long all = __ballot(ol >= 0 && tl > kP2Own);
+    while (all) {
+        const int r = __builtin_ctzll(all);
+        all &= all - 1;
+        longer(ib - wave * niw + r, __builtin_amdgcn_readlane(tl, r),
+               __builtin_amdgcn_readlane(ol, r), s_rows, (int)threadIdx.x, 256,
+               [] { __syncthreads(); });
         if (NN) {
-            const int b = wave_nearest(br2, bj);
-            if (lane == r) best = b;
+            if (lane == 0) {
+                s_br2[wave] = br2;
+                s_bj[wave] = bj;
+            }
+            __syncthreads();
+            if (wave == r / niw && lane == r % niw) {
+                double m2 = INFINITY;
+                int mj = INT_MAX;
+#pragma unroll
+                for (int w = 0; w < 4; ++w)
+                    if (s_br2[w] < m2 || (s_br2[w] == m2 && s_bj[w] < mj)) {
+                        m2 = s_br2[w];
+                        mj = s_bj[w];
+                    }
+                best = mj == INT_MAX ? -1 : mj;
+            }
         }
     }
 
@@ -1393,11 +1476,13 @@ void launch_jget(hipStream_t st, int n, const JRec *jp, double *x, double *v) {
 }
 
 void launch_copy_to_host(hipStream_t st, const void *src, void *dst,
-                         size_t bytes, const unsigned *err, unsigned *herr) {
+                         size_t bytes, size_t fixed, const int *nlast,
+                         const unsigned *err, unsigned *herr) {
     const size_t n16 = bytes / 16;
     const int nb = (int)std::min<size_t>(1024, std::max<size_t>(1, (n16 + 255) / 256));
     hipLaunchKernelGGL(k_copy_to_host, dim3(nb), dim3(256), 0, st,
-                       (const uint4 *)src, (uint4 *)dst, n16, err, herr);
+                       (const uint4 *)src, (uint4 *)dst, n16, fixed, nlast,
+                       err, herr);
 }
 
 void launch_copy_from_host(hipStream_t st, const void *src, void *dst,
