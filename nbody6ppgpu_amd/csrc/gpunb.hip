@@ -179,6 +179,8 @@ struct SortedView {
         v.nj = nj;
         v.ntile = ntile;
         v.blk0 = 0;
+        v.src = 0;
+        v.pad = 0;
         launch_set_prepclus(st, pc.p, v);
         prepare(st, jp, 1, prep_stat_blocks(nj), ntile);
     }
@@ -1158,8 +1160,15 @@ struct Ens {
     DevBuf<JStats> jst;
     HostBuf<double> h_send;
     DevBuf<double> d_send;
+    HostBuf<PrepClus> h_pc;
+    hipEvent_t ev_send = nullptr;   // after the uploads of the last send
+    bool ev_send_live = false;
     HostBuf<ClusterDesc> h_desc;
     DevBuf<ClusterDesc> d_desc;
+    // What d_desc and d_xr hold: an unchanged table is not uploaded again
+    // (an upload waits for the stream, the pinned copy may be in use).
+    std::vector<ClusterDesc> desc_up;
+    std::vector<long long> xr_up;
     DevBuf<double> part;
     DevBuf<int> nbc;   // zero between launches, as the engine's
     DevBuf<int> nbl;
@@ -1205,8 +1214,12 @@ void ens_close() {
     E.jst.release();
     E.h_send.release();
     E.d_send.release();
+    E.h_pc.release();
+    E.ev_send_live = false;
     E.h_desc.release();
     E.d_desc.release();
+    E.desc_up.clear();
+    E.xr_up.clear();
     E.part.release();
     E.nbc.release();
     E.nbl.release();
@@ -1266,41 +1279,44 @@ void ens_send(int ncl, const int *nj, const double *m, const double (*x)[3],
                 "gpunb_ens_send: nj outside 0..nbmax of the cluster");
         tot += nj[c];
     }
-    HIPCHK(hipStreamSynchronize(S.st));   // staging and graphs may be in use
+    // The pinned buffers may still be read by the previous send's uploads;
+    // everything on the device follows in stream order.
+    wait_event(E.ev_send, E.ev_send_live);
+    if (!E.ev_send)
+        HIPCHK(hipEventCreateWithFlags(&E.ev_send, hipEventDisableTiming));
     E.h_send.ensure(std::max<size_t>(7 * (size_t)tot, 7));
     E.d_send.ensure(std::max<size_t>(7 * (size_t)tot, 7));
+    E.h_pc.ensure((size_t)ncl);
     memcpy(E.h_send.p, m, tot * sizeof(double));
     memcpy(E.h_send.p + tot, x, 3 * tot * sizeof(double));
     memcpy(E.h_send.p + 4 * tot, v, 3 * tot * sizeof(double));
-    HIPCHK(hipMemcpyAsync(E.d_send.p, E.h_send.p, 7 * tot * sizeof(double),
-                          hipMemcpyHostToDevice, S.st));
-    launch_stats_reset(S.st, E.jst.p, nullptr);
-    long long o = 0;
-    for (int c = 0; c < ncl; ++c) {
-        const int pad = std::max(round_up(nj[c], kTile), round_up(E.nj[c], kTile));
-        launch_pack_j(S.st, E.d_send.p + o, E.d_send.p + tot + 3 * o,
-                      E.d_send.p + 4 * tot + 3 * o, nj[c], pad,
-                      E.jp.p + E.j0[c], E.jst.p, S.err.p);
-        E.nj[c] = nj[c];
-        o += nj[c];
-    }
     // Sorted view of every cluster: each one's whole capacity range (its
     // spare records are padding and sort last), so the ranges tile the
     // array.
-    std::vector<PrepClus> pcs((size_t)ncl);
-    int blk = 0;
+    int blk = 0, o = 0;
     for (int c = 0; c < ncl; ++c) {
-        pcs[c].j0 = E.j0[c];
-        pcs[c].nj = nj[c];
-        pcs[c].ntile = (c + 1 < ncl ? E.j0[c + 1] : E.jcap - kTile) / kTile -
-                       E.j0[c] / kTile;
-        pcs[c].blk0 = blk;
+        PrepClus &P = E.h_pc.p[c];
+        P.j0 = E.j0[c];
+        P.nj = nj[c];
+        P.ntile = (c + 1 < ncl ? E.j0[c + 1] : E.jcap - kTile) / kTile -
+                  E.j0[c] / kTile;
+        P.blk0 = blk;
+        P.src = o;
+        P.pad = std::max(round_up(nj[c], kTile), round_up(E.nj[c], kTile));
         blk += prep_stat_blocks(nj[c]);
+        o += nj[c];
+        E.nj[c] = nj[c];
     }
-    HIPCHK(hipMemcpyAsync(E.sv.pc.p, pcs.data(), ncl * sizeof(PrepClus),
+    HIPCHK(hipMemcpyAsync(E.d_send.p, E.h_send.p, 7 * tot * sizeof(double),
                           hipMemcpyHostToDevice, S.st));
+    HIPCHK(hipMemcpyAsync(E.sv.pc.p, E.h_pc.p, ncl * sizeof(PrepClus),
+                          hipMemcpyHostToDevice, S.st));
+    HIPCHK(hipEventRecord(E.ev_send, S.st));
+    E.ev_send_live = true;
+    launch_stats_reset(S.st, E.jst.p, nullptr);
+    launch_pack_clusters(S.st, E.sv.pc.p, ncl, E.jcap - kTile, E.d_send.p,
+                         (size_t)tot, E.jp.p, E.jst.p, S.err.p);
     E.sv.prepare(S.st, E.jp.p, ncl, blk, (E.jcap - kTile) / kTile);
-    HIPCHK(hipStreamSynchronize(S.st));   // pcs leaves scope
     HIPCHK(hipGetLastError());
 }
 
@@ -1413,9 +1429,7 @@ void ens_regf_dev(int ncl, const int *ni, const double *h2, const double *dtr,
         return;
     }
     // Cluster table, one entry per cluster; scratch offsets in cluster order.
-    HIPCHK(hipStreamSynchronize(S.st));   // the table may be in use
-    E.h_desc.ensure((size_t)ncl);
-    E.d_desc.ensure((size_t)ncl);
+    std::vector<ClusterDesc> table((size_t)ncl);
     std::vector<ClusterDesc> cd((size_t)ncl);
     long long pairs = 0, i0 = 0, work = 0;
     for (int c = 0; c < ncl; ++c) {
@@ -1466,7 +1480,7 @@ void ens_regf_dev(int ncl, const int *ni, const double *h2, const double *dtr,
         task += (long long)D.n_iw * D.nslice;
         blk += cdiv(D.ni, D.ipb);
         cost_all += (double)D.n_iw * D.nslice * tiles_per_task(order[k]);
-        E.h_desc.p[k] = D;
+        table[k] = D;
     }
     long long xr[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     {
@@ -1496,17 +1510,25 @@ void ens_regf_dev(int ncl, const int *ni, const double *h2, const double *dtr,
         launch_zero_int(S.st, E.nbc.p, (int)E.nbc.n);
         E.nbc_dirty = false;
     }
-    HIPCHK(hipMemcpyAsync(E.d_desc.p, E.h_desc.p, ncl * sizeof(ClusterDesc),
-                          hipMemcpyHostToDevice, S.st));
-    if (persist) {
-        E.queue.ensure(8);
-        E.d_xr.ensure(9);
+    const std::vector<long long> xrv(xr, xr + 9);
+    if (E.desc_up.size() != table.size() || E.xr_up != xrv ||
+        memcmp(E.desc_up.data(), table.data(), ncl * sizeof(ClusterDesc))) {
+        HIPCHK(hipStreamSynchronize(S.st));   // the pinned copies may be in use
+        E.desc_up.clear();
+        E.h_desc.ensure((size_t)ncl);
+        E.d_desc.ensure((size_t)ncl);
         E.h_xr.ensure(9);
+        E.d_xr.ensure(9);
+        memcpy(E.h_desc.p, table.data(), ncl * sizeof(ClusterDesc));
         memcpy(E.h_xr.p, xr, sizeof xr);
+        HIPCHK(hipMemcpyAsync(E.d_desc.p, E.h_desc.p, ncl * sizeof(ClusterDesc),
+                              hipMemcpyHostToDevice, S.st));
         HIPCHK(hipMemcpyAsync(E.d_xr.p, E.h_xr.p, sizeof xr,
                               hipMemcpyHostToDevice, S.st));
+        E.desc_up = table;
+        E.xr_up = xrv;
     }
-    HIPCHK(hipStreamSynchronize(S.st));
+    if (persist) E.queue.ensure(8);
     RegfLaunch R;
     memset(&R, 0, sizeof R);
     R.jps = E.sv.jps.p;

@@ -89,12 +89,15 @@ constexpr float kTileBand = 0.5f;
 
 // Cluster of a j preparation: j range [j0, j0 + ntile * kTile) of the
 // original and sorted arrays (tile aligned), nj real j at its start, and its
-// first statistics block.
+// first statistics block.  For launch_pack_clusters: its first body in the
+// sent arrays, and the records written (nj and padding).
 struct PrepClus {
     int j0;
     int nj;
     int ntile;
     int blk0;
+    int src;
+    int pad;
 };
 
 // Buffers of the sorted j view (one per engine; the ensemble has its own).
@@ -214,6 +217,11 @@ struct RegfLaunch {
 void launch_pack_j(hipStream_t st, const double *m, const double *x,
                    const double *v, int nj, int nj_pad, JRec *jp, JStats *jst,
                    unsigned *err);
+// The same for ncl clusters (device table pc, ranges tiling [0, n_all)) whose
+// tot bodies follow each other in the sent arrays m[tot], x[tot][3], v[tot][3].
+void launch_pack_clusters(hipStream_t st, const PrepClus *pc, int ncl,
+                          int n_all, const double *sent, size_t tot, JRec *jp,
+                          JStats *jst, unsigned *err);
 void launch_stats_reset(hipStream_t st, JStats *jst, int *total);
 void launch_predict(hipStream_t st, double t, int nj, int nj_pad,
                     const double *x0, const double *v0, const double *f,

@@ -145,12 +145,13 @@ __global__ void k_stats_reset(JStats *jst, int *total) {
     }
 }
 
-__global__ __launch_bounds__(256) void k_pack_j(
-    const double *__restrict__ m, const double *__restrict__ x,
-    const double *__restrict__ v, int nj, int nj_pad, JRec *__restrict__ jp,
-    JStats *__restrict__ jst, unsigned *__restrict__ err) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    double vmag = 0.0, mpos = INFINITY;
+// Record j of nj (padding up to nj_pad) -> *jp; its |v| and positive mass.
+__device__ inline void pack_record(const double *__restrict__ m,
+                                   const double *__restrict__ x,
+                                   const double *__restrict__ v, int j, int nj,
+                                   int nj_pad, JRec *__restrict__ jp,
+                                   unsigned *__restrict__ err, double &vmag,
+                                   double &mpos) {
     if (j < nj) {
         JRec r;
         r.x = x[3 * (size_t)j + 0];
@@ -164,13 +165,45 @@ __global__ __launch_bounds__(256) void k_pack_j(
         r.pad = 0.0f;
         const double chk = r.x + r.y + r.z + r.vx + r.vy + r.vz + r.m;
         if (chk != chk) atomicOr(err, ERR_NAN_J);
-        jp[j] = r;
+        *jp = r;
         vmag = speed_up(r.vx, r.vy, r.vz);
         if (r.m > 0.0) mpos = r.m;
     } else if (j < nj_pad) {
         JRec r;
         set_pad(r);
-        jp[j] = r;
+        *jp = r;
+    }
+}
+
+__global__ __launch_bounds__(256) void k_pack_j(
+    const double *__restrict__ m, const double *__restrict__ x,
+    const double *__restrict__ v, int nj, int nj_pad, JRec *__restrict__ jp,
+    JStats *__restrict__ jst, unsigned *__restrict__ err) {
+    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    double vmag = 0.0, mpos = INFINITY;
+    pack_record(m, x, v, j, nj, nj_pad, jp + j, err, vmag, mpos);
+    stats_fold(jst, vmag, mpos);
+}
+
+// Every cluster of an ensemble in one launch (24 clusters, a launch each: 24
+// times 4 us).
+__global__ __launch_bounds__(256) void k_pack_clusters(
+    const PrepClus *__restrict__ pc, int ncl, int n_all,
+    const double *__restrict__ sent, size_t tot, JRec *__restrict__ jp,
+    JStats *__restrict__ jst, unsigned *__restrict__ err) {
+    const int g = blockIdx.x * blockDim.x + threadIdx.x;
+    double vmag = 0.0, mpos = INFINITY;
+    if (g < n_all) {
+        int lo = 0, hi = ncl - 1;
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (pc[mid].j0 <= g) lo = mid;
+            else hi = mid - 1;
+        }
+        const PrepClus P = pc[lo];
+        pack_record(sent + P.src, sent + tot + 3 * (size_t)P.src,
+                    sent + 4 * tot + 3 * (size_t)P.src, g - P.j0, P.nj, P.pad,
+                    jp + g, err, vmag, mpos);
     }
     stats_fold(jst, vmag, mpos);
 }
@@ -1450,6 +1483,14 @@ void launch_pack_j(hipStream_t st, const double *m, const double *x,
     if (nj_pad <= 0) return;
     hipLaunchKernelGGL(k_pack_j, dim3(cdiv(nj_pad, 256)), dim3(256), 0, st, m,
                        x, v, nj, nj_pad, jp, jst, err);
+}
+
+void launch_pack_clusters(hipStream_t st, const PrepClus *pc, int ncl,
+                          int n_all, const double *sent, size_t tot, JRec *jp,
+                          JStats *jst, unsigned *err) {
+    if (n_all <= 0) return;
+    hipLaunchKernelGGL(k_pack_clusters, dim3(cdiv(n_all, 256)), dim3(256), 0, st,
+                       pc, ncl, n_all, sent, tot, jp, jst, err);
 }
 
 void launch_predict(hipStream_t st, double t, int nj, int nj_pad,
