@@ -104,8 +104,6 @@ struct SortedView {
     DevBuf<PrepClus> pc;
     DevBuf<unsigned long long> kin, kout;
     DevBuf<int> vin, vout;
-    DevBuf<char> tmp;
-    size_t tmp_bytes = 0;
     DevBuf<double> part;
 
     // cap_j records (a whole number of tiles including one spare tile past
@@ -132,14 +130,13 @@ struct SortedView {
         kout.release();
         vin.release();
         vout.release();
-        tmp.release();
-        tmp_bytes = 0;
         part.release();
     }
     // Enqueue the preparation of ncl clusters whose table (pc, device) is in
-    // place: they tile [0, ntile_all * kTile) and hold nblk statistics blocks.
+    // place: they tile [0, ntile_all * kTile), at most ntile_max tiles each, and
+    // hold nblk statistics blocks.
     void prepare(hipStream_t st, const JRec *jp, int ncl, int nblk,
-                 int ntile_all) {
+                 int ntile_all, int ntile_max) {
         if (ntile_all <= 0) return;
         const size_t n = (size_t)ntile_all * kTile;
         kin.ensure(n);
@@ -147,12 +144,6 @@ struct SortedView {
         vin.ensure(n);
         vout.ensure(n);
         part.ensure(8 * (size_t)nblk);
-        const size_t need = jprep_tmp_bytes((int)n, ncl);
-        if (need == 0) throw Error("j preparation: sort storage query failed");
-        if (need > tmp_bytes) {
-            tmp.ensure(need);
-            tmp_bytes = need;
-        }
         JView V;
         V.jp = jp;
         V.jps = jps.p;
@@ -165,10 +156,8 @@ struct SortedView {
         B.key_out = kout.p;
         B.val_in = vin.p;
         B.val_out = vout.p;
-        B.tmp = tmp.p;
-        B.tmp_bytes = tmp_bytes;
         B.part = part.p;
-        HIPCHK(launch_jprep(st, V, pc.p, ncl, nblk, ntile_all, B));
+        HIPCHK(launch_jprep(st, V, pc.p, ncl, nblk, ntile_all, ntile_max, B));
     }
     // One cluster covering [0, round_up(nj, kTile)).
     void prepare_one(hipStream_t st, const JRec *jp, int nj) {
@@ -182,7 +171,7 @@ struct SortedView {
         v.src = 0;
         v.pad = 0;
         launch_set_prepclus(st, pc.p, v);
-        prepare(st, jp, 1, prep_stat_blocks(nj), ntile);
+        prepare(st, jp, 1, prep_stat_blocks(nj), ntile, ntile);
     }
 };
 
@@ -233,8 +222,6 @@ struct State {
     // storage and the i data gathered into that order.
     DevBuf<unsigned> ikey_in, ikey_out;
     DevBuf<int> ival_in, iperm;
-    DevBuf<char> itmp;
-    size_t itmp_bytes = 0;
     DevBuf<double> isorted;   // xs [ni][3], vs [ni][3], hs [ni], ds [ni]
     hipStream_t st2 = nullptr;
     hipEvent_t ev_p1[2] = {nullptr, nullptr}, ev_p2[2] = {nullptr, nullptr};
@@ -573,19 +560,11 @@ void enqueue_regf(int ni, const double *xi, const double *vi, const double *h2,
         S.ival_in.ensure(n);
         S.iperm.ensure(n);
         S.isorted.ensure(8 * n);
-        const size_t need = isort_tmp_bytes(ni);
-        if (need == 0) throw Error("i sort: storage query failed");
-        if (need > S.itmp_bytes) {
-            S.itmp.ensure(need);
-            S.itmp_bytes = need;
-        }
         ISortBufs B = {};
         B.key_in = S.ikey_in.p;
         B.key_out = S.ikey_out.p;
         B.val_in = S.ival_in.p;
         B.perm = S.iperm.p;
-        B.tmp = S.itmp.p;
-        B.tmp_bytes = S.itmp_bytes;
         B.xs = S.isorted.p;
         B.vs = B.xs + 3 * n;
         B.hs = B.vs + 3 * n;
@@ -853,8 +832,6 @@ void do_close() {
     S.ikey_out.release();
     S.ival_in.release();
     S.iperm.release();
-    S.itmp.release();
-    S.itmp_bytes = 0;
     S.isorted.release();
     S.d_res.release();
     S.h_res.release();
@@ -1183,8 +1160,6 @@ struct Ens {
     // permutation, gathered i data, and the clusters' i starts.
     DevBuf<unsigned long long> ikey_in, ikey_out;
     DevBuf<int> ival_in, iperm, d_i0;
-    DevBuf<char> itmp;
-    size_t itmp_bytes = 0;
     DevBuf<double> isorted;
     HostBuf<int> h_i0;
     std::vector<int> i0_up;   // the starts last uploaded to d_i0
@@ -1228,8 +1203,6 @@ void ens_close() {
     E.ival_in.release();
     E.iperm.release();
     E.d_i0.release();
-    E.itmp.release();
-    E.itmp_bytes = 0;
     E.isorted.release();
     E.h_i0.release();
     E.i0_up.clear();
@@ -1293,7 +1266,7 @@ void ens_send(int ncl, const int *nj, const double *m, const double (*x)[3],
     // Sorted view of every cluster: each one's whole capacity range (its
     // spare records are padding and sort last), so the ranges tile the
     // array.
-    int blk = 0, o = 0;
+    int blk = 0, o = 0, ntile_max = 0;
     for (int c = 0; c < ncl; ++c) {
         PrepClus &P = E.h_pc.p[c];
         P.j0 = E.j0[c];
@@ -1303,6 +1276,7 @@ void ens_send(int ncl, const int *nj, const double *m, const double (*x)[3],
         P.blk0 = blk;
         P.src = o;
         P.pad = std::max(round_up(nj[c], kTile), round_up(E.nj[c], kTile));
+        ntile_max = std::max(ntile_max, P.ntile);
         blk += prep_stat_blocks(nj[c]);
         o += nj[c];
         E.nj[c] = nj[c];
@@ -1316,7 +1290,7 @@ void ens_send(int ncl, const int *nj, const double *m, const double (*x)[3],
     launch_stats_reset(S.st, E.jst.p, nullptr);
     launch_pack_clusters(S.st, E.sv.pc.p, ncl, E.jcap - kTile, E.d_send.p,
                          (size_t)tot, E.jp.p, E.jst.p, S.err.p);
-    E.sv.prepare(S.st, E.jp.p, ncl, blk, (E.jcap - kTile) / kTile);
+    E.sv.prepare(S.st, E.jp.p, ncl, blk, (E.jcap - kTile) / kTile, ntile_max);
     HIPCHK(hipGetLastError());
 }
 
@@ -1384,25 +1358,17 @@ void ens_regf_dev(int ncl, const int *ni, const double *h2, const double *dtr,
         E.ival_in.ensure(n);
         E.iperm.ensure(n);
         E.isorted.ensure(8 * n);
-        const size_t need = isort_ens_tmp_bytes((int)n, ncl);
-        if (need == 0) throw Error("ensemble i sort: storage query failed");
-        if (need > E.itmp_bytes) {
-            E.itmp.ensure(need);
-            E.itmp_bytes = need;
-        }
         ISortBufs B = {};
         B.key64_in = E.ikey_in.p;
         B.key64_out = E.ikey_out.p;
         B.val_in = E.ival_in.p;
         B.perm = E.iperm.p;
-        B.tmp = E.itmp.p;
-        B.tmp_bytes = E.itmp_bytes;
         B.xs = E.isorted.p;
         B.vs = B.xs + 3 * n;
         B.hs = B.vs + 3 * n;
         B.ds = B.hs + n;
         HIPCHK(launch_isort_ens(S.st, E.sv.jcl.p, E.d_i0.p, ncl, xi, vi, h2, dtr,
-                                (int)n, B));
+                                (int)n, *std::max_element(ni, ni + ncl), B));
         xi = B.xs;
         vi = B.vs;
         h2 = B.hs;

@@ -235,7 +235,7 @@ void launch_jget(hipStream_t st, int n, const JRec *jp, double *x, double *v);
 // j preparation (jprep.hip): per-cluster statistics, Hilbert sort and the
 // records of the sorted view, for ncl clusters whose ranges (device table pc)
 // tile [0, ntile_all * kTile).  nblk = sum over clusters of
-// prep_stat_blocks(nj).
+// prep_stat_blocks(nj), ntile_max the largest cluster's ntile.
 constexpr int kStatChunk = 2048;   // j per statistics block
 inline int prep_stat_blocks(int nj) {
     return nj > 0 ? (nj + kStatChunk - 1) / kStatChunk : 1;
@@ -243,36 +243,29 @@ inline int prep_stat_blocks(int nj) {
 struct PrepBufs {
     unsigned long long *key_in, *key_out;
     int *val_in, *val_out;
-    void *tmp;
-    size_t tmp_bytes;
     double *part;      // 8 doubles per statistics block
 };
-// rocprim temporary storage for sorting n keys of ncl clusters.
-size_t jprep_tmp_bytes(int n, int ncl);
 hipError_t launch_jprep(hipStream_t st, const JView &V, const PrepClus *pc,
-                        int ncl, int nblk, int ntile_all, const PrepBufs &B);
+                        int ncl, int nblk, int ntile_all, int ntile_max,
+                        const PrepBufs &B);
 // Hilbert order of the i of one call (jprep.hip): perm[p] = the original i
 // at sorted position p, and the i data gathered into that order.
 struct ISortBufs {
     unsigned *key_in, *key_out;                 // one cluster (32-bit keys)
     unsigned long long *key64_in, *key64_out;   // ensemble (cluster << 32 | code)
     int *val_in, *perm;
-    void *tmp;
-    size_t tmp_bytes;
     double *xs, *vs, *hs, *ds;   // [ni][3], [ni][3], [ni], [ni]
 };
-size_t isort_tmp_bytes(int n);
 hipError_t launch_isort(hipStream_t st, const JClus *jcl, const double *xi,
                         const double *vi, const double *h2, const double *dtr,
                         int ni, const ISortBufs &B);
 // Ensemble: the i of every cluster in Hilbert order within the cluster (its
 // range [cl_i0[c], cl_i0[c + 1]) of the concatenated i kept), keyed in the
-// box of the cluster's j set.
-size_t isort_ens_tmp_bytes(int n, int ncl);
+// box of the cluster's j set.  ni_max: the largest cluster's i.
 hipError_t launch_isort_ens(hipStream_t st, const JClus *jcl, const int *cl_i0,
                             int ncl, const double *xi, const double *vi,
                             const double *h2, const double *dtr, int ni,
-                            const ISortBufs &B);
+                            int ni_max, const ISortBufs &B);
 // *pc = v, in stream order.
 void launch_set_prepclus(hipStream_t st, PrepClus *pc, const PrepClus &v);
 // Padding records in j32[0, n) and empty tiles in tiles[0, ntile).

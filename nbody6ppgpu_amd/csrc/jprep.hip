@@ -12,17 +12,15 @@
 //              in a fixed order
 //   k_jstat2   per cluster: the blocks' partials in block order -> JClus
 //              (bounding box, mean mass)
-//   k_jkey     64-bit keys (cluster << 32 | heavy << 30 | 30-bit Hilbert index
-//              of the position in the cluster's box; padding records sort
-//              last)
-//   rocprim radix sort of (key, original index): stable, so equal codes keep
-//              their index order
+//   sort       by key (cluster << 32 | heavy << 30 | 30-bit Hilbert index of
+//              the position in the cluster's box; padding records sort last),
+//              stable, so equal codes keep their index order: k_sort_runs,
+//              then k_sort_merge once or more
 //   k_jtile    one wavefront per tile: sorted FP64 records, sorted -> original
 //              index map, tile centres and offset bounds, FP32 records
 #include "gpunb_internal.h"
 
-#include <rocprim/device/device_radix_sort.hpp>
-
+#include <algorithm>
 #include <cfloat>
 #include <cmath>
 
@@ -218,26 +216,385 @@ __global__ __launch_bounds__(256) void k_jstat2(const PrepClus *__restrict__ pc,
     }
 }
 
-__global__ __launch_bounds__(256) void k_jkey(
-    const JRec *__restrict__ jp, const PrepClus *__restrict__ pc, int ncl,
-    const JClus *__restrict__ jcl, int n_all, unsigned long long *__restrict__ key,
-    int *__restrict__ val) {
-    const int g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= n_all) return;
-    const int c = clus_of(pc, ncl, g);
-    const PrepClus P = pc[c];
-    const JClus &J = jcl[c];
-    unsigned code = 0xffffffffu;       // padding records sort last
-    if (g - P.j0 < P.nj) {
-        const JRec &r = jp[g];
-        code = cell_key(r.x, r.y, r.z, J);
-        // Heavy bodies (m > kHeavy <m>) sort after the light ones, in tiles
-        // of their own: their band weight w_j would otherwise widen the
-        // near region of every tile that holds one.
-        if (r.m > (double)kHeavy * J.mbar) code |= 1u << 30;
+// Key code of record g of cluster c, and of an i in the box of J.
+__device__ inline unsigned j_code(const JRec *__restrict__ jp, const PrepClus &P,
+                                  const JClus &J, int g) {
+    if (g - P.j0 >= P.nj) return 0xffffffffu;       // padding sorts last
+    const JRec &r = jp[g];
+    unsigned code = cell_key(r.x, r.y, r.z, J);
+    // Heavy bodies (m > kHeavy <m>) sort after the light ones, in tiles of
+    // their own: their band weight w_j would otherwise widen the near region
+    // of every tile that holds one.
+    if (r.m > (double)kHeavy * J.mbar) code |= 1u << 30;
+    return code;
+}
+__device__ inline unsigned i_code(const double *__restrict__ xi, const JClus &J,
+                                  int g) {
+    return cell_key(xi[3 * (size_t)g + 0], xi[3 * (size_t)g + 1],
+                    xi[3 * (size_t)g + 2], J);
+}
+// Cluster of global i g: the last c with cl_i0[c] <= g (clusters hold
+// consecutive i ranges in cluster order, empty ones repeat the next start).
+__device__ inline int iclus_of(const int *__restrict__ cl_i0, int ncl, int g) {
+    int lo = 0, hi = ncl - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (cl_i0[mid] <= g) lo = mid;
+        else hi = mid - 1;
     }
-    key[g] = ((unsigned long long)c << 32) | code;
-    val[g] = g;
+    return lo;
+}
+
+// ---------------------------------------------------------------------------
+// Stable sort.  k_sort_runs sorts runs of kSortRun consecutive records by
+// (cluster, code) in LDS, forming the keys itself; k_sort_merge merges up to
+// kSortWay runs in one launch, and the last merge writes the result (for i:
+// gathers the data) in place of another launch.
+//
+// Bound: launches, load latency and cold instructions, not bandwidth (a sort
+// of N = 16411 moves 0.4 MB).  The library's radix sort is at these sizes a
+// block sort and a launch per doubling, 8 launches and 41 us for N = 16411
+// besides the key and gather launches; here 12.2 + 18.0 us with the keys in
+// them (131072: 45 us before, 12.8 + 28.6 + 25.6 us).  Whole step, j and i
+// sorts: N = 9000 435 -> 423 us, 16411 703 -> 688 us, 32000 1480 -> 1450 us,
+// 131072 13.63 -> 13.66 ms (within its spread).  Rolled loops: unrolled ones
+// are 11 KB of code that every launch fetches for one pass, 26.5 us for the
+// merge and 703 -> 707 us.
+// ---------------------------------------------------------------------------
+constexpr int kSortRun = 1024;   // records of a first run, one per thread
+constexpr int kSortWay = 32;     // runs of one merge
+
+struct JSort32 {      // j records of one cluster
+    using Key = unsigned;
+    const JRec *jp;
+    const PrepClus *pc;
+    const JClus *jcl;
+    int *out;
+    __device__ Key key(int g) const { return j_code(jp, pc[0], jcl[0], g); }
+    __device__ void range(Key, int n, int &b, int &e) const { b = 0, e = n; }
+    __device__ void put(int p, int g) const { out[p] = g; }
+};
+struct JSort64 {      // j records of an ensemble
+    using Key = unsigned long long;
+    const JRec *jp;
+    const PrepClus *pc;
+    const JClus *jcl;
+    int *out;
+    int ncl;
+    __device__ Key key(int g) const {
+        const int c = clus_of(pc, ncl, g);
+        return ((Key)c << 32) | j_code(jp, pc[c], jcl[c], g);
+    }
+    __device__ void range(Key k, int, int &b, int &e) const {
+        const PrepClus &P = pc[k >> 32];
+        b = P.j0;
+        e = P.j0 + P.ntile * kTile;
+    }
+    __device__ void put(int p, int g) const { out[p] = g; }
+};
+// Hilbert order of the i of a call in the box of their cluster's j set, so
+// that the 64 i of a pass-1 wavefront are spatially close: far tiles then skip
+// the screen for the whole wave, and the near band's FP64 pairs gather in
+// fewer tiles.  The i data are gathered into that order.
+struct IGather {
+    const double *xi, *vi, *h2, *dtr;
+    double *xs, *vs, *hs, *ds;
+    int *perm;
+    __device__ void put(int p, int i) const {
+        perm[p] = i;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            xs[3 * (size_t)p + c] = xi[3 * (size_t)i + c];
+            vs[3 * (size_t)p + c] = vi[3 * (size_t)i + c];
+        }
+        hs[p] = h2[i];
+        ds[p] = dtr[i];
+    }
+};
+struct ISort32 : IGather {
+    using Key = unsigned;
+    const JClus *jcl;
+    __device__ Key key(int g) const { return i_code(xi, jcl[0], g); }
+    __device__ void range(Key, int n, int &b, int &e) const { b = 0, e = n; }
+};
+struct ISort64 : IGather {
+    using Key = unsigned long long;
+    const JClus *jcl;
+    const int *cl_i0;
+    int ncl;
+    __device__ Key key(int g) const {
+        const int c = iclus_of(cl_i0, ncl, g);
+        return ((Key)c << 32) | i_code(xi, jcl[c], g);
+    }
+    __device__ void range(Key k, int, int &b, int &e) const {
+        b = cl_i0[k >> 32];
+        e = cl_i0[(k >> 32) + 1];
+    }
+};
+
+// One record per thread; each level a record finds its place in the pair of
+// sorted pieces of w by binary search in the other piece (equal keys: the
+// first piece's before the second's).
+template <class S>
+__global__ __launch_bounds__(kSortRun) void k_sort_runs(S s, int n,
+                                                        typename S::Key *__restrict__ key,
+                                                        int *__restrict__ val) {
+    using Key = typename S::Key;
+    __shared__ Key lk[2][kSortRun];
+    __shared__ unsigned short lv[2][kSortRun];
+    const int t = threadIdx.x;
+    const int g = blockIdx.x * kSortRun + t;
+    lk[0][t] = g < n ? s.key(g) : ~(Key)0;     // past the end: sorts last
+    lv[0][t] = (unsigned short)t;
+    __syncthreads();
+#pragma unroll 1
+    for (int w = 1, cur = 0; w < kSortRun; w <<= 1, cur ^= 1) {
+        const Key k = lk[cur][t];
+        const bool second = (t & w) != 0;
+        const int pair = t & ~(2 * w - 1);
+        const int other = pair + (second ? 0 : w);
+        int pos = 0;                 // of 0..w - 1; the last record below
+#pragma unroll 1
+        for (int h = w >> 1; h >= 1; h >>= 1) {
+            const Key o = lk[cur][other + pos + h - 1];
+            pos += (second ? o <= k : o < k) ? h : 0;
+        }
+        const Key o = lk[cur][other + pos];
+        pos += (second ? o <= k : o < k) ? 1 : 0;
+        const int d = pair + (t & (w - 1)) + pos;
+        lk[cur ^ 1][d] = k;
+        lv[cur ^ 1][d] = lv[cur][t];
+        __syncthreads();
+    }
+    constexpr int last = __builtin_ctz(kSortRun) & 1;
+    if (g < n) {
+        key[g] = lk[last][t];
+        val[g] = blockIdx.x * kSortRun + lv[last][t];
+    }
+}
+
+// Records among a[0, m) (ascending) before one of key k: the smaller keys,
+// and the equal ones where eq.  8 pieces a step: their ends' loads overlap,
+// a halving search would wait for each (1024 records: 4 waits, not 10).
+template <class Key>
+__host__ __device__ inline int count_before(const Key *a, int m, Key k, bool eq) {
+    int lo = 0, len = m;             // the count is in [lo, lo + len]
+    while (len > 0) {
+        const int st = (len + 7) >> 3;
+        int c = 0;
+#pragma unroll
+        for (int u = 1; u < 8; ++u) {
+            const bool in = u * st <= len;
+            const Key o = a[lo + (in ? u * st : st) - 1];
+            c += (in && (eq ? o <= k : o < k)) ? 1 : 0;
+        }
+        const bool closed = c < 7 && (c + 1) * st <= len;   // probe c + 1 is not before
+        lo += c * st;
+        len = closed ? st - 1 : len - c * st;
+    }
+    return lo;
+}
+
+// A workgroup places 64 consecutive records of a run of L among the runs
+// r0..r1: the records of every other run that lie between the first and the
+// last of them are counted for each by search in LDS, those before the first
+// are common.  kSortWay / kParts runs a wavefront, so that its loads are in
+// flight together.
+constexpr int kParts = 4;
+constexpr int kPartWay = kSortWay / kParts;
+template <class Key>
+struct MergeLds {
+    static constexpr int kWin = 16384 / (int)sizeof(Key);
+    Key win[kWin + 1];               // one more: read for an empty window
+    int cnt[2 * kSortWay];           // records before the first, the last
+    int off[kSortWay + 1];           // windows' starts in win, their total
+    int common;
+    int sum[kParts][64];
+};
+// Steps of the threads t, a barrier between each.
+template <class Key>
+__host__ __device__ inline void merge_windows(MergeLds<Key> &S, int t,
+                                              const Key *key, int n, long long L,
+                                              int own, int r0, int r1, Key first,
+                                              Key last) {
+    if (t >= 2 * kSortWay) return;
+    const int r = r0 + (t >> 1);
+    int c = 0;
+    if (r <= r1 && r != own) {
+        const long long a = r * L;
+        c = count_before(key + a, (int)(n - a < L ? n - a : L),
+                         (t & 1) ? last : first, r < own);
+    }
+    S.cnt[t] = c;
+}
+template <class Key>
+__host__ __device__ inline void merge_offsets(MergeLds<Key> &S, int t) {
+    if (t > kSortWay) return;
+    int sum = 0, common = 0;
+#pragma unroll 8
+    for (int q = 0; q < kSortWay; ++q) {
+        const int lo = S.cnt[2 * q], hi = S.cnt[2 * q + 1];
+        sum += q < t ? hi - lo : 0;
+        common += lo;
+    }
+    S.off[t] = sum;
+    if (t == 0) S.common = common;
+}
+template <class Key>
+__host__ __device__ inline void merge_load(MergeLds<Key> &S, int t,
+                                           const Key *key, long long L, int r0) {
+    if (S.off[kSortWay] > MergeLds<Key>::kWin) return;   // searched in place
+    const int lane = t & 63, q0 = (t >> 6) * kPartWay;
+    Key v[kPartWay][2];
+    int w[kPartWay];
+#pragma unroll
+    for (int u = 0; u < kPartWay; ++u) {
+        const int q = q0 + u;
+        const Key *a = key + (r0 + q) * L + S.cnt[2 * q];
+        w[u] = S.off[q + 1] - S.off[q];
+        if (lane < w[u]) v[u][0] = a[lane];
+        if (lane + 64 < w[u]) v[u][1] = a[lane + 64];
+    }
+#pragma unroll
+    for (int u = 0; u < kPartWay; ++u) {
+        const int q = q0 + u;
+        if (lane < w[u]) S.win[S.off[q] + lane] = v[u][0];
+        if (lane + 64 < w[u]) S.win[S.off[q] + lane + 64] = v[u][1];
+        for (int e = lane + 128; e < w[u]; e += 64)
+            S.win[S.off[q] + e] = key[(r0 + q) * L + S.cnt[2 * q] + e];
+    }
+}
+// Records of part `part` in the windows before one of key k; at(q, e, w) is
+// the e-th of window q of w, anything past it.
+template <class Key, class At>
+__host__ __device__ inline int merge_count(const MergeLds<Key> &S, int part, int own,
+                                           int r0, Key k, At at) {
+    int pos[kPartWay], w[kPartWay], wmax = 0;
+    const int q0 = part * kPartWay;
+#pragma unroll
+    for (int u = 0; u < kPartWay; ++u) {
+        pos[u] = 0;
+        w[u] = S.off[q0 + u + 1] - S.off[q0 + u];
+        wmax = w[u] > wmax ? w[u] : wmax;
+    }
+    if (wmax == 0) return 0;
+    for (int h = 1 << (31 - __builtin_clz(wmax)); h >= 1; h >>= 1)
+#pragma unroll
+        for (int u = 0; u < kPartWay; ++u) {
+            const int e = pos[u] + h - 1;
+            const Key o = at(q0 + u, e, w[u]);
+            const bool before = r0 + q0 + u < own ? o <= k : o < k;
+            pos[u] += e < w[u] && before ? h : 0;
+        }
+    int sum = 0;
+#pragma unroll
+    for (int u = 0; u < kPartWay; ++u) sum += pos[u];
+    return sum;
+}
+template <class Key>
+__host__ __device__ inline void merge_ranks(MergeLds<Key> &S, int t, const Key *key,
+                                            long long L, int own, int r0, Key k) {
+    const int part = t >> 6;
+    int c;
+    if (S.off[kSortWay] <= MergeLds<Key>::kWin)
+        c = merge_count(S, part, own, r0, k,
+                        [&](int q, int e, int w) {
+                            return S.win[S.off[q] + (e < w ? e : 0)];
+                        });
+    else
+        c = merge_count(S, part, own, r0, k, [&](int q, int e, int w) {
+            return e < w ? key[(r0 + q) * L + S.cnt[2 * q] + e] : (Key)0;
+        });
+    S.sum[part][t & 63] = c;
+}
+// Place of the group's record `lane`, at position p.
+template <class Key>
+__host__ __device__ inline int merge_place(const MergeLds<Key> &S, int lane,
+                                           long long L, int own, int r0, int p) {
+    int d = (int)(r0 * L + (p - own * L)) + S.common;
+#pragma unroll
+    for (int part = 0; part < kParts; ++part) d += S.sum[part][lane];
+    return d;
+}
+
+// One merge of runs of L, a workgroup per 64 records.  kLast: runs of the
+// records' whole clusters, at most kSortWay, the result put by S; else
+// kSortWay runs at a time.
+template <class S, bool kLast>
+__global__ __launch_bounds__(64 * kParts) void k_sort_merge(S s, int n, int L,
+                                                   const typename S::Key *__restrict__ key,
+                                                   const int *__restrict__ val,
+                                                   typename S::Key *__restrict__ key_out,
+                                                   int *__restrict__ val_out) {
+    using Key = typename S::Key;
+    __shared__ MergeLds<Key> lds;
+    const int t = threadIdx.x, lane = t & 63;
+    const int p0 = blockIdx.x * 64;
+    const int p1 = min(p0 + 63, n - 1);
+    const int p = min(p0 + lane, p1);
+    const int own = p0 / L;
+    const Key first = key[p0], last = key[p1], k = key[p];
+    const int v = val[p];
+    int r0, r1;
+    if constexpr (kLast) {
+        int beg, end, x;
+        s.range(first, n, beg, x);
+        s.range(last, n, x, end);
+        r0 = beg / L;
+        r1 = (end - 1) / L;
+    } else {
+        r0 = own & ~(kSortWay - 1);
+        r1 = min(r0 + kSortWay - 1, (n - 1) / L);
+    }
+    merge_windows(lds, t, key, n, (long long)L, own, r0, r1, first, last);
+    __syncthreads();
+    merge_offsets(lds, t);
+    __syncthreads();
+    merge_load(lds, t, key, (long long)L, r0);
+    __syncthreads();
+    merge_ranks(lds, t, key, (long long)L, own, r0, k);
+    __syncthreads();
+    if (t >= 64 || p0 + t > p1) return;
+    const int d = merge_place(lds, lane, (long long)L, own, r0, p);
+    if constexpr (kLast) {
+        s.put(d, v);
+    } else {
+        key_out[d] = k;
+        val_out[d] = v;
+    }
+}
+
+// Sort of n records, a cluster holding at most n_max of them, in the buffers
+// A and B; s.put may write B's values.
+template <class S>
+static hipError_t sort_records(hipStream_t st, const S &s, int n, int n_max,
+                               bool one, typename S::Key *key_a, int *val_a,
+                               typename S::Key *key_b, int *val_b) {
+    // The last merge takes the runs of whole clusters.  64 records of a run
+    // can be of several: the first's may begin, the last's end, span - 1 runs
+    // away, so a cluster spans at most half of kSortWay; a single one all.
+    auto final_at = [&](long long L) {
+        return one ? (n + L - 1) / L <= kSortWay : (n_max - 1) / L + 2 <= kSortWay / 2;
+    };
+    int merges = 0;
+    for (long long L = kSortRun; !final_at(L); L *= kSortWay) ++merges;
+    if (merges & 1) {             // the last merge reads A
+        std::swap(key_a, key_b);
+        std::swap(val_a, val_b);
+    }
+    hipLaunchKernelGGL((k_sort_runs<S>), dim3((n + kSortRun - 1) / kSortRun),
+                       dim3(kSortRun), 0, st, s, n, key_a, val_a);
+    const dim3 grid((n + 63) / 64);
+    long long L = kSortRun;
+    for (; merges > 0; --merges, L *= kSortWay) {
+        hipLaunchKernelGGL((k_sort_merge<S, false>), grid, dim3(64 * kParts), 0, st, s, n,
+                           (int)L, key_a, val_a, key_b, val_b);
+        std::swap(key_a, key_b);
+        std::swap(val_a, val_b);
+    }
+    hipLaunchKernelGGL((k_sort_merge<S, true>), grid, dim3(64 * kParts), 0, st, s, n,
+                       (int)L, key_a, val_a, key_b, val_b);
+    return hipGetLastError();
 }
 
 __global__ __launch_bounds__(64) void k_jtile(
@@ -345,126 +702,28 @@ __global__ __launch_bounds__(256) void k_park_view(JRec32 *__restrict__ j32,
     }
 }
 
-static unsigned key_bits(int ncl) {
-    unsigned cbits = 0;
-    while ((1 << cbits) < ncl) ++cbits;
-    return 32u + cbits;
-}
-
-// Hilbert order of the i of a call in the j set's box (cluster 0), so that
-// the 64 i of a pass-1 wavefront are spatially close: far tiles then skip
-// the screen for the whole wave, and the near band's FP64 pairs gather in
-// fewer tiles.
-__global__ __launch_bounds__(256) void k_ikey(const double *__restrict__ xi,
-                                              int ni, const JClus *__restrict__ jcl,
-                                              unsigned *__restrict__ key,
-                                              int *__restrict__ val) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= ni) return;
-    key[i] = cell_key(xi[3 * (size_t)i + 0], xi[3 * (size_t)i + 1],
-                      xi[3 * (size_t)i + 2], jcl[0]);
-    val[i] = i;
-}
-
-// The i data in sorted order: xs/vs [ni][3], hs/ds [ni].
-__global__ __launch_bounds__(256) void k_igather(
-    const int *__restrict__ perm, int ni, const double *__restrict__ xi,
-    const double *__restrict__ vi, const double *__restrict__ h2,
-    const double *__restrict__ dtr, double *__restrict__ xs,
-    double *__restrict__ vs, double *__restrict__ hs, double *__restrict__ ds) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= ni) return;
-    const int i = perm[p];
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        xs[3 * (size_t)p + c] = xi[3 * (size_t)i + c];
-        vs[3 * (size_t)p + c] = vi[3 * (size_t)i + c];
-    }
-    hs[p] = h2[i];
-    ds[p] = dtr[i];
-}
-
-// Ensemble i keys: (cluster << 32) | Hilbert index of x_i in the box of the
-// cluster owning global i (the last c with cl_i0[c] <= i; clusters hold
-// consecutive i ranges in cluster order, empty ones repeat the next start).
-__global__ __launch_bounds__(256) void k_ikey_ens(
-    const double *__restrict__ xi, int ni, const int *__restrict__ cl_i0,
-    int ncl, const JClus *__restrict__ jcl, unsigned long long *__restrict__ key,
-    int *__restrict__ val) {
-    const int g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= ni) return;
-    int lo = 0, hi = ncl - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (cl_i0[mid] <= g) lo = mid;
-        else hi = mid - 1;
-    }
-    const unsigned code = cell_key(xi[3 * (size_t)g + 0], xi[3 * (size_t)g + 1],
-                                   xi[3 * (size_t)g + 2], jcl[lo]);
-    key[g] = ((unsigned long long)lo << 32) | code;
-    val[g] = g;
-}
-
-size_t isort_ens_tmp_bytes(int n, int ncl) {
-    size_t bytes = 0;
-    const hipError_t rc = rocprim::radix_sort_pairs(
-        nullptr, bytes, (const unsigned long long *)nullptr,
-        (unsigned long long *)nullptr, (const int *)nullptr, (int *)nullptr,
-        (size_t)std::max(n, 1), 0u, key_bits(ncl), (hipStream_t)0);
-    return rc == hipSuccess ? bytes : 0;
-}
-
 hipError_t launch_isort_ens(hipStream_t st, const JClus *jcl, const int *cl_i0,
                             int ncl, const double *xi, const double *vi,
                             const double *h2, const double *dtr, int ni,
-                            const ISortBufs &B) {
+                            int ni_max, const ISortBufs &B) {
     if (ni <= 0) return hipSuccess;
-    const dim3 g((ni + 255) / 256);
-    hipLaunchKernelGGL(k_ikey_ens, g, dim3(256), 0, st, xi, ni, cl_i0, ncl, jcl,
-                       B.key64_in, B.val_in);
-    size_t bytes = B.tmp_bytes;
-    const hipError_t rc = rocprim::radix_sort_pairs(
-        B.tmp, bytes, B.key64_in, B.key64_out, B.val_in, B.perm, (size_t)ni, 0u,
-        key_bits(ncl), st);
-    if (rc != hipSuccess) return rc;
-    hipLaunchKernelGGL(k_igather, g, dim3(256), 0, st, B.perm, ni, xi, vi, h2,
-                       dtr, B.xs, B.vs, B.hs, B.ds);
-    return hipGetLastError();
-}
-
-size_t isort_tmp_bytes(int n) {
-    size_t bytes = 0;
-    const hipError_t rc = rocprim::radix_sort_pairs(
-        nullptr, bytes, (const unsigned *)nullptr, (unsigned *)nullptr,
-        (const int *)nullptr, (int *)nullptr, (size_t)std::max(n, 1), 0u, 30u,
-        (hipStream_t)0);
-    return rc == hipSuccess ? bytes : 0;
+    ISort64 s;
+    static_cast<IGather &>(s) = {xi, vi, h2, dtr, B.xs, B.vs, B.hs, B.ds, B.perm};
+    s.jcl = jcl;
+    s.cl_i0 = cl_i0;
+    s.ncl = ncl;
+    return sort_records(st, s, ni, ni_max, ncl == 1, B.key64_in, B.val_in,
+                        B.key64_out, B.perm);
 }
 
 hipError_t launch_isort(hipStream_t st, const JClus *jcl, const double *xi,
                         const double *vi, const double *h2, const double *dtr,
                         int ni, const ISortBufs &B) {
     if (ni <= 0) return hipSuccess;
-    const dim3 g((ni + 255) / 256);
-    hipLaunchKernelGGL(k_ikey, g, dim3(256), 0, st, xi, ni, jcl, B.key_in,
-                       B.val_in);
-    size_t bytes = B.tmp_bytes;
-    const hipError_t rc = rocprim::radix_sort_pairs(
-        B.tmp, bytes, B.key_in, B.key_out, B.val_in, B.perm, (size_t)ni, 0u, 30u,
-        st);
-    if (rc != hipSuccess) return rc;
-    hipLaunchKernelGGL(k_igather, g, dim3(256), 0, st, B.perm, ni, xi, vi, h2,
-                       dtr, B.xs, B.vs, B.hs, B.ds);
-    return hipGetLastError();
-}
-
-size_t jprep_tmp_bytes(int n, int ncl) {
-    size_t bytes = 0;
-    const hipError_t rc = rocprim::radix_sort_pairs(
-        nullptr, bytes, (const unsigned long long *)nullptr,
-        (unsigned long long *)nullptr, (const int *)nullptr, (int *)nullptr,
-        (size_t)std::max(n, 1), 0u, key_bits(ncl), (hipStream_t)0);
-    return rc == hipSuccess ? bytes : 0;
+    ISort32 s;
+    static_cast<IGather &>(s) = {xi, vi, h2, dtr, B.xs, B.vs, B.hs, B.ds, B.perm};
+    s.jcl = jcl;
+    return sort_records(st, s, ni, ni, true, B.key_in, B.val_in, B.key_out, B.perm);
 }
 
 void launch_set_prepclus(hipStream_t st, PrepClus *pc, const PrepClus &v) {
@@ -480,19 +739,24 @@ void launch_park_view(hipStream_t st, JRec32 *j32, int n, JTile *tiles,
 }
 
 hipError_t launch_jprep(hipStream_t st, const JView &V, const PrepClus *pc,
-                        int ncl, int nblk, int ntile_all, const PrepBufs &B) {
+                        int ncl, int nblk, int ntile_all, int ntile_max,
+                        const PrepBufs &B) {
     if (ntile_all <= 0) return hipSuccess;
     const int n_all = ntile_all * kTile;
     hipLaunchKernelGGL(k_jstat1, dim3(nblk), dim3(256), 0, st, V.jp, pc, ncl,
                        B.part);
     hipLaunchKernelGGL(k_jstat2, dim3(ncl), dim3(256), 0, st, pc, ncl, nblk,
                        B.part, V.jcl);
-    hipLaunchKernelGGL(k_jkey, dim3((n_all + 255) / 256), dim3(256), 0, st, V.jp,
-                       pc, ncl, V.jcl, n_all, B.key_in, B.val_in);
-    size_t bytes = B.tmp_bytes;
-    const hipError_t rc = rocprim::radix_sort_pairs(
-        B.tmp, bytes, B.key_in, B.key_out, B.val_in, B.val_out, (size_t)n_all,
-        0u, key_bits(ncl), st);
+    hipError_t rc;
+    if (ncl == 1) {
+        const JSort32 k = {V.jp, pc, V.jcl, B.val_out};
+        rc = sort_records(st, k, n_all, n_all, true, (unsigned *)B.key_in, B.val_in,
+                          (unsigned *)B.key_out, B.val_out);
+    } else {
+        const JSort64 k = {V.jp, pc, V.jcl, B.val_out, ncl};
+        rc = sort_records(st, k, n_all, ntile_max * kTile, false, B.key_in, B.val_in,
+                          B.key_out, B.val_out);
+    }
     if (rc != hipSuccess) return rc;
     hipLaunchKernelGGL(k_jtile, dim3(ntile_all), dim3(64), 0, st, V.jp, pc, ncl,
                        V.jcl, B.val_out, V.jps, V.j32, V.tiles, V.jidx);
