@@ -513,8 +513,8 @@ __device__ inline double again(double v) {
 // kIBlockMin i-wavefronts, the wavefronts are instead cut into eight blocks of
 // consecutive ones, taken block by block and slice by slice within a block:
 // XCD x then runs every slice for one eighth of the i, in Hilbert order.
-// The King N = 131072 launch takes 13.8 ms that way against 15.0 ms
-// slice-major, with the same results; ensembles and small calls (1024 i)
+// The King N = 131072 launch took 13.8 ms that way against 15.0 ms
+// slice-major (12.4 ms now, the order unchanged), with the same results; ensembles and small calls (1024 i)
 // measured slower, so they keep slice-major order.
 constexpr int kIBlocks = 8;
 constexpr int kIBlockMin = 256;
@@ -1142,7 +1142,7 @@ __global__ __launch_bounds__(64 * kP1W, p1_waves(G)) void k_regf_pass1_f64_q(
 //
 // Bound: latency (a wavefront's chain of dependent loads).  Before, an i at a
 // time with lanes over the slices, every entry ranked against all others:
-// 1024 i of N = 15565 with mass-weighted lists 190 us, now 42 us; 114k i of
+// 1024 i of N = 15565 with mass-weighted lists 190 us, now 35 us; 114k i of
 // 24 clusters 360 -> 90 us; 1024 i of N = 131072 16.5 -> 11 us.
 //
 // The nearest neighbour (NN; smallest FP64 r2 > 0, ties to the smaller j) is
