@@ -410,18 +410,28 @@ int pick_group() {
     return 2;
 }
 
-double pick_rounds(int ni) {
+double pick_rounds(int ni, double most) {
     if (S.rounds > 0) return S.rounds;
     const char *r = getenv("GPUNB_WAVE_ROUNDS");
     if (r && atof(r) > 0) return atof(r);
     // Resident-wave capacity multiples per launch, by block size: large
-    // blocks take up to 12 (King N = 131072 in one launch, whole step:
-    // 16.96 ms at 6, 16.32 at 12, 16.74 at 24), small ones fewer, since
-    // every extra slice is one more FP64 partial per i to write and reduce
-    // (whole step, 1024 i: 0.187 ms at 1, 0.206 at 4; 128 i: 0.108 ms at
-    // 0.5, 0.121 at 4).  1024 scattered i through gpunb_regf_: 5.05e11
-    // pairs/s at 0.75, 5.3e11 at 1, 5.2e11 at 1.5, 5.4e11 at 2.
-    return std::min(12.0, std::max(0.5, ni / 512.0));
+    // blocks take up to `most`, small ones fewer, since every extra slice is
+    // one more FP64 partial per i to write and reduce (whole step, 1024 i:
+    // 0.187 ms at 1, 0.206 at 4; 128 i: 0.108 ms at 0.5, 0.121 at 4).  1024
+    // scattered i through gpunb_regf_: 5.05e11 pairs/s at 0.75, 5.3e11 at 1,
+    // 5.2e11 at 1.5, 5.4e11 at 2.
+    return std::min(most, std::max(0.5, ni / 512.0));
+}
+// Most rounds.  Ensembles: 24 clusters 2.04 ms at 12, 2.08 at 24; 64 clusters
+// 5.61 and 5.56.
+constexpr double kRounds = 12.0;
+// One cluster: as many up to 65536 i (King, whole step: N = 32000 1.445 ms at
+// 12, 1.478 at 6; 65536 4.19 at 12, 4.17 at 24), then in proportion to ni:
+// the last round is the launch's idle end, and a wavefront still has about 30
+// tiles (90000 7.36 ms at 12, 7.31 at 16; 131072 13.52 at 12,
+// 13.27 at 24, 13.23 at 32 and 48; Plummer 12.42, 12.04, 12.12, 12.16).
+double most_rounds(int ni) {
+    return std::max(kRounds, ni * (24.0 / 131072.0));
 }
 
 // Pair arithmetic of a call.  Default: the mixed kernel (32) when the i run
@@ -453,7 +463,8 @@ int resident_waves(int m_flag, int group, int prec) {
 // tile each take slices down to one unit per wavefront.
 int decompose(int ni_c, int ntile, int m_flag, int group, int prec, int &ju) {
     const int n_iw = cdiv(ni_c, 64);
-    const double target = resident_waves(m_flag, group, prec) * pick_rounds(ni_c);
+    const double target = resident_waves(m_flag, group, prec) *
+                          pick_rounds(ni_c, most_rounds(ni_c));
     ju = prec >= 64 ? 4 : 6;
     const bool fine = prec >= 64 && (long long)n_iw * ntile < 1024;
     const int nu = fine ? ntile << (6 - ju) : ntile;
@@ -1302,7 +1313,7 @@ int ens_slice_tiles(const int *ni, int group, int prec, int m_flag) {
     for (int c = 0; c < E.ncl; ++c) ni_all += ni[c];
     const double target =
         resident_waves(m_flag, group, prec) *
-        pick_rounds((int)std::min<long long>(ni_all, 1 << 30));
+        pick_rounds((int)std::min<long long>(ni_all, 1 << 30), kRounds);
     int lo = 1, hi = 1024;
     auto waves = [&](int L) {
         double w = 0;
