@@ -514,7 +514,7 @@ __device__ inline double again(double v) {
 // consecutive ones, taken block by block and slice by slice within a block:
 // XCD x then runs every slice for one eighth of the i, in Hilbert order.
 // The King N = 131072 launch took 13.8 ms that way against 15.0 ms
-// slice-major (12.4 ms now, the order unchanged), with the same results; ensembles and small calls (1024 i)
+// slice-major (12.2 ms now, the order unchanged), with the same results; ensembles and small calls (1024 i)
 // measured slower, so they keep slice-major order.
 constexpr int kIBlocks = 8;
 constexpr int kIBlockMin = 256;
