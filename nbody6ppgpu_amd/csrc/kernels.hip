@@ -616,7 +616,11 @@ __device__ __forceinline__ void regf_pass1_task(
         const double pzd = dz + dtrd * dvz;
         const double r2pd = sq3d(pxd, pyd, pzd);
         const double mnd = r2d < r2pd ? r2d : r2pd;
-        const double H = MFLAG ? J.m * h2[i] : h2[i];
+        // A lane past the last i has no h2 and takes no list entry: its
+        // position (0, 0, 0) can be a body's, which the mass-weighted screen
+        // flags.
+        const double h2d = act ? h2[i] : 0.0;
+        const double H = MFLAG ? J.m * h2d : h2d;
         if ((mnd < H) && (j < nj)) {
             hit.push(j);
         } else if (r2d != 0.0) {
@@ -929,7 +933,8 @@ __device__ __forceinline__ void regf_pass1_f64_task(
         const double pzd = dz + dtrd * dvz;
         const double r2pd = sq3d(pxd, pyd, pzd);
         const double mnd = r2d < r2pd ? r2d : r2pd;
-        const double H = MFLAG ? J.m * h2[i] : h2[i];
+        const double h2d = act ? h2[i] : 0.0;   // none past the last i
+        const double H = MFLAG ? J.m * h2d : h2d;
         if ((mnd < H) && (j < nj)) {
             hit.push(j);
         } else if (r2d != 0.0) {
