@@ -1183,7 +1183,10 @@ struct Ens {
 Ens E;
 
 void ens_graph_drop() {
-    if (E.gexec) (void)hipGraphExecDestroy(E.gexec);
+    if (E.gexec) {
+        HIPCHK(hipStreamSynchronize(S.st));   // its last launch may still run
+        (void)hipGraphExecDestroy(E.gexec);
+    }
     if (E.graph) (void)hipGraphDestroy(E.graph);
     E.gexec = nullptr;
     E.graph = nullptr;
