@@ -290,8 +290,7 @@ struct DBuf {
     size_t cap = 0;
     void ensure(size_t n) {
         if (n <= cap) return;
-        if (p) (void)hipFree(p);
-        p = nullptr;
+        release();
         ICHK(hipMalloc((void **)&p, std::max<size_t>(n, 1) * sizeof(T)));
         cap = n;
     }
@@ -308,8 +307,7 @@ struct HBuf {
     size_t cap = 0;
     void ensure(size_t n) {
         if (n <= cap) return;
-        if (p) (void)hipHostFree(p);
-        p = nullptr;
+        release();
         ICHK(hipHostMalloc((void **)&p, std::max<size_t>(n, 1) * sizeof(T)));
         cap = n;
     }
@@ -511,7 +509,8 @@ void split(size_t n, size_t bytes, F f) {
     for (int k = 0; k < started; ++k) th[k].join();
 }
 
-// A block that can hold what *want says, from the idle ones or new.
+// A block that can hold n records, or n rows of nflat members in all, from the
+// idle ones or new.
 Block *take_block(bool rows, int n, size_t nflat) {
     Block *b = nullptr;
     if (!I.idle.empty()) {
@@ -570,6 +569,22 @@ void place_block(Block *b) {
     }
 }
 
+// Stage a block that fill fills.  After an error nothing of it is staged: it is
+// at rest, and what it was to hold stays where the caller has it.
+template <class F>
+void stage_block(bool rows, int n, size_t nflat, F fill) {
+    I.blocks.reserve(I.blocks.size() + 1);
+    Block *b = take_block(rows, n, nflat);
+    try {
+        fill(b);
+        place_block(b);
+    } catch (...) {
+        I.idle.push_back(b);
+        throw;
+    }
+    I.blocks.push_back(b);
+}
+
 // Whether a batched call of n bodies is staged as a block (lock held).
 bool block_ok(int n) {
     if (n < kBlockMin || I.blocks.size() >= kMaxBlocks) return false;
@@ -606,9 +621,7 @@ bool block_jp(int n, const int *addr, const double *x, const double *v,
               const double *t0) {
     std::lock_guard<std::mutex> g(g_stage_mu);
     if (!block_ok(n) || !addresses_once(n, addr)) return false;
-    Block *b = take_block(false, n, 0);
-    I.blocks.push_back(b);
-    try {
+    stage_block(false, n, 0, [&](Block *b) {
         double *h = b->soa();
         int *slot = b->ints();
         const size_t N = (size_t)n;
@@ -621,12 +634,7 @@ bool block_jp(int n, const int *addr, const double *x, const double *v,
             memcpy(h + 13 * N + lo, t0 + lo, (hi - lo) * sizeof(double));
             for (size_t q = lo; q < hi; ++q) slot[q] = addr[q] - 1;
         });
-        place_block(b);
-    } catch (...) {
-        I.blocks.pop_back();
-        I.idle.push_back(b);
-        throw;
-    }
+    });
     return true;
 }
 
@@ -639,9 +647,7 @@ bool block_lists(int n, const int *addr, const int *nnb, const int *members) {
         nf += (size_t)nnb[q];
     }
     if (nf > (size_t)INT_MAX || !addresses_once(n, addr)) return false;
-    Block *b = take_block(true, n, nf);
-    I.blocks.push_back(b);
-    try {
+    stage_block(true, n, nf, [&](Block *b) {
         int *hdr = b->ints(), *flat = hdr + 3 * (size_t)n;
         int off = 0;
         for (int q = 0; q < n; ++q) {
@@ -663,13 +669,8 @@ bool block_lists(int n, const int *addr, const int *nnb, const int *members) {
             if (out) pbad->store(true, std::memory_order_relaxed);
         });
         IREQ(!bad.load(), "list member out of range [1, nmax]");
-        place_block(b);
-        for (int q = 0; q < n; ++q) I.nnb[addr[q] - 1] = nnb[q];
-    } catch (...) {
-        I.blocks.pop_back();
-        I.idle.push_back(b);
-        throw;
-    }
+    });
+    for (int q = 0; q < n; ++q) I.nnb[addr[q] - 1] = nnb[q];
     return true;
 }
 
@@ -677,22 +678,21 @@ bool block_lists(int n, const int *addr, const int *nnb, const int *members) {
 void block_merged() {
     const size_t nj = I.jp_rec.size();
     if (nj) {
-        Block *b = take_block(false, (int)nj, 0);
-        I.blocks.push_back(b);
-        double *h = b->soa();
-        for (size_t k = 0; k < nj; ++k) {
-            const IRec &r = I.jp_rec[k];
-            for (int c = 0; c < 3; ++c) {
-                h[3 * k + c] = r.x[c];
-                h[3 * (nj + k) + c] = r.v[c];
-                h[3 * (2 * nj + k) + c] = r.f[c];
-                h[3 * (3 * nj + k) + c] = r.fd[c];
+        stage_block(false, (int)nj, 0, [&](Block *b) {
+            double *h = b->soa();
+            for (size_t k = 0; k < nj; ++k) {
+                const IRec &r = I.jp_rec[k];
+                for (int c = 0; c < 3; ++c) {
+                    h[3 * k + c] = r.x[c];
+                    h[3 * (nj + k) + c] = r.v[c];
+                    h[3 * (2 * nj + k) + c] = r.f[c];
+                    h[3 * (3 * nj + k) + c] = r.fd[c];
+                }
+                h[12 * nj + k] = r.m;
+                h[13 * nj + k] = r.t0;
             }
-            h[12 * nj + k] = r.m;
-            h[13 * nj + k] = r.t0;
-        }
-        memcpy(b->ints(), I.jp_addr.data(), nj * sizeof(int));
-        place_block(b);
+            memcpy(b->ints(), I.jp_addr.data(), nj * sizeof(int));
+        });
         for (int s : I.jp_addr) I.jp_slot[s] = -1;
         I.jp_rec.clear();
         I.jp_addr.clear();
@@ -700,17 +700,17 @@ void block_merged() {
     size_t nr = 0;
     for (size_t r = 0; r < I.ls_hdr.size(); r += 3) nr += I.ls_hdr[r] >= 0;
     if (nr) {
-        Block *b = take_block(true, (int)nr, I.ls_flat.size());
-        I.blocks.push_back(b);
-        int *hdr = b->ints();
+        stage_block(true, (int)nr, I.ls_flat.size(), [&](Block *b) {
+            int *hdr = b->ints();
+            for (size_t r = 0; r < I.ls_hdr.size(); r += 3)
+                if (I.ls_hdr[r] >= 0) {
+                    memcpy(hdr, I.ls_hdr.data() + r, 3 * sizeof(int));
+                    hdr += 3;
+                }
+            memcpy(hdr, I.ls_flat.data(), I.ls_flat.size() * sizeof(int));
+        });
         for (size_t r = 0; r < I.ls_hdr.size(); r += 3)
-            if (I.ls_hdr[r] >= 0) {
-                memcpy(hdr, I.ls_hdr.data() + r, 3 * sizeof(int));
-                hdr += 3;
-                I.ls_slot[I.ls_hdr[r]] = -1;
-            }
-        memcpy(hdr, I.ls_flat.data(), I.ls_flat.size() * sizeof(int));
-        place_block(b);
+            if (I.ls_hdr[r] >= 0) I.ls_slot[I.ls_hdr[r]] = -1;
     }
     I.ls_hdr.clear();
     I.ls_flat.clear();

@@ -16,6 +16,7 @@ PREAMBLE = """
 import ctypes, sys
 stub = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
 stub.stub_most_device.argtypes = [ctypes.c_size_t]
+stub.stub_most_pinned.argtypes = [ctypes.c_size_t]
 stub.stub_held_device.restype = ctypes.c_size_t
 import numpy as np
 from nbody6ppgpu_amd import gpunb
@@ -76,4 +77,65 @@ def test_graph_is_not_destroyed_while_it_runs(stub):
         ensemble.call(other, [100, 70], 20)
         gpunb.gpunb_ens_close()
         assert stub.stub_graph_faults() == 0, stub.stub_graph_faults()
+    """)
+
+
+IRR = """
+    n = 6000
+    gpunb.irr_open(n, 40)
+    idx = np.arange(n)
+    x = np.zeros((n, 3))
+    m = np.zeros(n)
+    rows = [np.array([1 + (i + 1) % n], np.int32) for i in range(n)]
+
+    def jp(s):
+        gpunb.irr_set_jp(s + 1, x[s], x[s], x[s], x[s], m[s], m[s])
+
+    def lists(s):
+        gpunb.irr_set_lists(s + 1, [rows[i] for i in s])
+"""
+
+
+def test_irr_refused_upload_stages_nothing(stub):
+    """Records and rows of per-particle calls whose upload finds no memory, or
+    fails: an error, and the next call sends them."""
+    run(stub, IRR + """
+    one = [np.array([i]) for i in range(3000)]
+    full = [np.arange(1, 31, dtype=np.int32)] * n
+    rows = full                                   # rows of 372 KB in all
+    for fault in ("memory", "copy"):
+        for s in one:
+            jp(s)
+            lists(s)
+        if fault == "memory":
+            stub.stub_most_device(200 << 10)
+        else:
+            stub.stub_fail_uploads(1)
+        assert refused(gpunb.irr_firr, 0.0, idx[:100] + 1)
+        stub.stub_most_device(1 << 40)
+        if fault == "copy":
+            for s in one:         # newer rows of the same bodies
+                lists(s)
+            stub.stub_fail_uploads(1)
+            assert refused(gpunb.irr_firr, 0.0, idx[:100] + 1)
+        gpunb.irr_firr(0.0, idx[:100] + 1)
+        assert stub.stub_null_args() == 0
+        assert stub.stub_launches(b"k_irr_stage") > 0
+    """)
+
+
+def test_irr_buffer_that_did_not_grow_is_not_used(stub):
+    """A batch that needs larger buffers than there is memory for is refused,
+    and smaller ones after it are staged in buffers of their own."""
+    run(stub, IRR + """
+    for limit, most in ((stub.stub_most_device, 5000), (stub.stub_most_pinned, 6000)):
+        jp(idx[:3000])
+        gpunb.irr_firr(0.0, idx[:10] + 1)
+        limit(116 * most - 1)
+        assert refused(jp, idx[:most])
+        limit(1 << 40)
+        jp(idx[:3000])
+        gpunb.irr_firr(0.0, idx[:10] + 1)
+        assert stub.stub_null_args() == 0
+    gpunb.irr_close()
     """)
