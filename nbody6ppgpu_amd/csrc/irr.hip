@@ -37,7 +37,6 @@
 #include <mutex>
 #include <stdexcept>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -501,8 +500,8 @@ void split(size_t n, size_t bytes, F f) {
                 th[started] = std::thread([=] { f(lo, hi); });
                 done = hi;
             }
-        } catch (const std::system_error &) {
-            // No more threads: this one does the rest.
+        } catch (const std::exception &) {
+            // No more threads, or no memory for one: this one does the rest.
         }
     }
     f(done, n);

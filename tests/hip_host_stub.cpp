@@ -12,6 +12,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <new>
 #include <string>
 
 namespace {
@@ -20,6 +21,7 @@ std::mutex mu;
 size_t most_device = SIZE_MAX;   // a larger hipMalloc fails
 size_t most_pinned = SIZE_MAX;   // a larger hipHostMalloc fails
 int fail_uploads = 0;            // that many host-to-device copies fail
+int fail_new = -1;               // operator new fails after so many calls
 size_t held_device = 0;          // bytes of device memory not freed
 bool graph_running = false;      // launched, and not waited for since
 int graph_faults = 0;            // executable graphs destroyed while running
@@ -63,6 +65,7 @@ extern "C" {
 void stub_most_device(size_t bytes) { most_device = bytes; }
 void stub_most_pinned(size_t bytes) { most_pinned = bytes; }
 void stub_fail_uploads(int n) { fail_uploads = n; }
+void stub_fail_new(int n) { fail_new = n; }
 size_t stub_held_device() { return held_device; }
 int stub_graph_faults() { return graph_faults; }
 int stub_null_args() { return null_args; }
@@ -238,3 +241,13 @@ const char *hipGetErrorString(hipError_t e) {
 }
 
 }  // extern "C"
+
+// The library's heap allocations come here too.
+void *operator new(size_t bytes) {
+    if (fail_new >= 0 && fail_new-- == 0) throw std::bad_alloc();
+    void *p = malloc(bytes ? bytes : 1);
+    if (!p) throw std::bad_alloc();
+    return p;
+}
+void operator delete(void *p) noexcept { free(p); }
+void operator delete(void *p, size_t) noexcept { free(p); }

@@ -139,3 +139,20 @@ def test_irr_buffer_that_did_not_grow_is_not_used(stub):
         assert stub.stub_null_args() == 0
     gpunb.irr_close()
     """)
+
+
+def test_irr_split_copy_without_memory_for_threads(stub):
+    """A batch whose copy is split over threads, with every allocation of the
+    call failing in its turn: staged or refused, the process going on."""
+    run(stub, IRR.replace("n = 6000", "n = 20000") + """
+    assert 116 * n >= 2 << 20
+    done = []
+    for k in range(12):
+        stub.stub_fail_new(k)
+        done.append(not refused(jp, idx))
+        stub.stub_fail_new(-1)
+        gpunb.irr_firr(0.0, idx[:10] + 1)
+        assert stub.stub_null_args() == 0
+    assert done[-1] and any(done[:6])
+    gpunb.irr_close()
+    """)
