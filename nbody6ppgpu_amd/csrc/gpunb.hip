@@ -300,6 +300,7 @@ int guarded(const char *fn, F &&f) {
         f();
         return 0;
     } catch (const std::exception &e) {
+        (void)hipGetLastError();   // reported here, not by the next call
         report(fn, e.what());
         return -1;
     }

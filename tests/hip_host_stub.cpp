@@ -26,6 +26,7 @@ size_t held_device = 0;          // bytes of device memory not freed
 bool graph_running = false;      // launched, and not waited for since
 int graph_faults = 0;            // executable graphs destroyed while running
 int null_args = 0;               // launches of k_irr_stage without its data
+hipError_t last_error = hipSuccess;
 std::map<void *, size_t> blocks;
 std::map<const void *, std::string> names;
 std::map<std::string, int> launches;
@@ -109,7 +110,7 @@ hipError_t hipExtLaunchKernel(const void *fn, dim3, dim3, void **args, size_t,
 hipError_t hipMalloc(void **p, size_t bytes) {
     std::lock_guard<std::mutex> g(mu);
     *p = bytes <= most_device ? take(bytes) : nullptr;
-    if (!*p) return hipErrorOutOfMemory;
+    if (!*p) return last_error = hipErrorOutOfMemory;
     blocks[*p] = bytes;
     held_device += bytes;
     return hipSuccess;
@@ -235,7 +236,11 @@ hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int *n, const void *, in
     *n = 4;
     return hipSuccess;
 }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() {
+    const hipError_t e = last_error;
+    last_error = hipSuccess;
+    return e;
+}
 const char *hipGetErrorString(hipError_t e) {
     return e == hipErrorOutOfMemory ? "out of memory" : "error";
 }
