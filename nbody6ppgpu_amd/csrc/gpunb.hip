@@ -67,6 +67,20 @@ struct DevBuf {
         HIPCHK(hipMalloc((void **)&p, bytes));
         n = need;
     }
+    // Whether there is memory for need; false leaves the buffer empty.
+    bool try_ensure(size_t need) {
+        if (need <= n) return true;
+        release();
+        const hipError_t rc = hipMalloc((void **)&p, need * sizeof(T));
+        if (rc == hipSuccess) {
+            n = need;
+            return true;
+        }
+        p = nullptr;
+        if (rc != hipErrorOutOfMemory) HIPCHK(rc);
+        (void)hipGetLastError();   // not the launches' that follow
+        return false;
+    }
     void release() {
         if (p) (void)hipFree(p);
         p = nullptr;
@@ -855,6 +869,9 @@ void do_close() {
     S.en_cpot.release();
     S.en_ckin.release();
     S.en_part.release();
+    S.pot_rec.release();
+    S.pot_m.release();
+    S.d_ppart.release();
     S.nbmax = 0;
     S.nj = 0;
     S.njp = 0;
@@ -1006,9 +1023,11 @@ void do_profile(int irank) {
 
 // Potential of bodies i0 .. i0 + ni - 1 over all n, device arrays.  All
 // bodies of a set of 4096 to 4M go through the kernel that forms each 1/r
-// once (its partials are 2 KiB a body at the upper end); below, its block
-// pairs would not fill the machine (N = 4096: 63 us a call, 67 with
-// k_pot_pass1; N = 16384: 143 and 167; N = 131072: 3.59 and 5.83 ms).
+// once; below, its block pairs would not fill the machine (N = 4096: 63 us a
+// call, 67 with k_pot_pass1; N = 16384: 143 and 167; N = 131072: 3.59 and 5.83
+// ms).  Its partials are the engine's largest workspace (0.54 GB at N =
+// 131072, 2.2 GB at 1M, 8.6 GB at 4M): without the memory for them the bodies
+// take the other kernel, which needs a few MB, and gpunb_close_ gives them back.
 void enqueue_pot(const double *d_m, const double *d_x, int n, int i0, int ni,
                  double *d_pot) {
     const int ntile = cdiv(n, kTile);
@@ -1019,10 +1038,11 @@ void enqueue_pot(const double *d_m, const double *d_x, int n, int i0, int ni,
                   S.err.p);
     if (i0 == 0 && ni == n && n >= 4096 && n <= (1 << 22)) {
         const PotSym P = pot_sym_plan(ntile);
-        S.d_ppart.ensure((size_t)(P.nblock + 1) * n_pad);
-        launch_pot_sym(S.st, S.pot_rec.p, S.pot_m.p, n, ntile, P, S.d_ppart.p,
-                       d_pot);
-        return;
+        if (S.d_ppart.try_ensure((size_t)(P.nblock + 1) * n_pad)) {
+            launch_pot_sym(S.st, S.pot_rec.p, S.pot_m.p, n, ntile, P,
+                           S.d_ppart.p, d_pot);
+            return;
+        }
     }
     if (!S.pot_resident) S.pot_resident = pot_resident_waves();
     const int target = std::max(S.pot_resident, 1024) * 2;

@@ -159,3 +159,26 @@ def test_irr_split_copy_without_memory_for_threads(stub):
         assert done
     gpunb.irr_close()
     """)
+
+
+def test_potential_without_memory_for_its_partials(stub):
+    """All bodies, with too little device memory for the partials of the
+    kernel that forms each 1/r once: the other kernel, not an error; and
+    gpunb_close_ gives the partials back."""
+    run(stub, """
+        n = 40000
+        m, x = np.ones(n), np.zeros((n, 3))
+        gpunb.gpunb_open(100)
+        held = stub.stub_held_device()
+        stub.stub_most_device(30 << 20)
+        gpunb.gpupot(1, n, m, x)
+        assert stub.stub_launches(b"k_pot_sym") == 0
+        assert stub.stub_launches(b"k_pot_pass1") == 1
+        stub.stub_most_device(1 << 40)
+        gpunb.gpupot(1, n, m, x)
+        assert stub.stub_launches(b"k_pot_sym") == 1
+        assert stub.stub_held_device() > held + (90 << 20)
+        gpunb.gpunb_close()
+        gpunb.gpunb_open(100)
+        assert stub.stub_held_device() < held + (4 << 20)
+    """)
