@@ -102,10 +102,6 @@ hipError_t hipLaunchKernel(const void *fn, dim3, dim3, void **args, size_t,
                            hipStream_t) {
     return launched(fn, args);
 }
-hipError_t hipExtLaunchKernel(const void *fn, dim3, dim3, void **args, size_t,
-                              hipStream_t, hipEvent_t, hipEvent_t, int) {
-    return launched(fn, args);
-}
 
 hipError_t hipMalloc(void **p, size_t bytes) {
     std::lock_guard<std::mutex> g(mu);
