@@ -182,3 +182,21 @@ def test_potential_without_memory_for_its_partials(stub):
         gpunb.gpunb_open(100)
         assert stub.stub_held_device() < held + (4 << 20)
     """)
+
+
+def test_irr_small_batches_share_scatter_launches(stub):
+    """Ten batches of a hundred bodies, records and lists, and one call: the
+    first batch of each kind and all others together, two launches.  Batches
+    large enough for the copy engine are a launch each."""
+    run(stub, IRR + """
+    for s in np.split(idx[:1000], 10):
+        jp(s)
+        lists(s)
+    gpunb.irr_firr(0.0, idx[:1000] + 1)
+    assert stub.stub_launches(b"k_irr_stage") == 2
+    for _ in range(3):
+        jp(idx)
+    gpunb.irr_firr(0.0, idx[:1000] + 1)
+    assert stub.stub_launches(b"k_irr_stage") == 2 + 3
+    gpunb.irr_close()
+    """)
