@@ -345,14 +345,19 @@ __global__ void k_zero_int(int *p, int n) {
     if (k < n) p[k] = 0;
 }
 
-// LDS of a pass-1 workgroup, one part per wavefront: while the pair loops
-// run it holds the list entries found (row k: entry k of every lane), after
-// them the wavefront's FP64 sums.  Both are kHitRows * 64 ints.
+// LDS of a pass-1 workgroup, one part per wavefront.  w: while the pair loops
+// run, the list entries found (row k: entry k of every lane), after them the
+// wavefront's FP64 sums.  Both are kHitRows * 64 ints.  h2: that of the lanes'
+// i for the exact predicate (a register more would cost the mixed kernel a
+// resident wavefront, a load from memory is a wait per flagged pair); 0 for a
+// lane past the last i, which takes no list entry: its position (0, 0, 0) can
+// be a body's, which the mass-weighted screen flags.
 constexpr int kHitRows = 14;
 static_assert(kHitRows * 64 * sizeof(int) == 7 * 64 * sizeof(double),
               "the list entries and the sums share a wavefront's LDS");
 struct alignas(16) P1Lds {
     int w[kP1W][kHitRows * 64];
+    double h2[kP1W][64];
 };
 
 // The list entries of one lane (i).  They are kept in LDS and appended to
@@ -379,9 +384,14 @@ struct HitList {
             n = 0;
         }
     }
-    __device__ __forceinline__ void push(int j) {
-        lds[64 * n] = j;
-        if (++n == kHitRows) flush();
+    // Needs room for one more: a full lane is flushed as it fills up (FP64
+    // kernel, scattered i: few lanes of a wavefront have entries at a time), or
+    // room is made for a group of pairs in all lanes together (mixed kernel:
+    // the lanes of nearby i fill up one after the other, and would be flushed
+    // at as many points of the loop).
+    __device__ __forceinline__ void push(int j) { lds[64 * n++] = j; }
+    __device__ __forceinline__ void make_room(int g) {
+        if (__ballot(n > kHitRows - g) != 0) flush();
     }
 };
 
@@ -574,6 +584,7 @@ __device__ __forceinline__ void regf_pass1_task(
     double x0 = 0.0, y0 = 0.0, z0 = 0.0, u0 = 0.0, w0 = 0.0, q0 = 0.0;
     double dtr2x = 0.0;         // 2 dtr
     double thr = -1.0;          // FP64 screen threshold (k_regf_pass1_f64)
+    lds.h2[wv][lane] = 0.0;     // read by the lane itself
     float adtr = 0.0f;          // >= |dtr|
     float B = 0.0f;             // band base
     float hrad = 0.0f;          // >= sqrt(h2) (sqrt(h2 <m>) mass-weighted)
@@ -585,6 +596,7 @@ __device__ __forceinline__ void regf_pass1_task(
         w0 = vi[3 * (size_t)i + 1];
         q0 = vi[3 * (size_t)i + 2];
         const double h2d = h2[i], dtrd = dtr[i];
+        lds.h2[wv][lane] = h2d;
         dtr2x = 2.0 * dtrd;
         const double chk = x0 + y0 + z0 + u0 + w0 + q0 + h2d + dtrd;
         if (chk != chk) atomicOr(err, ERR_NAN_I);
@@ -616,10 +628,7 @@ __device__ __forceinline__ void regf_pass1_task(
         const double pzd = dz + dtrd * dvz;
         const double r2pd = sq3d(pxd, pyd, pzd);
         const double mnd = r2d < r2pd ? r2d : r2pd;
-        // A lane past the last i has no h2 and takes no list entry: its
-        // position (0, 0, 0) can be a body's, which the mass-weighted screen
-        // flags.
-        const double h2d = act ? h2[i] : 0.0;
+        const double h2d = lds.h2[wv][lane];
         const double H = MFLAG ? J.m * h2d : h2d;
         if ((mnd < H) && (j < nj)) {
             hit.push(j);
@@ -756,7 +765,8 @@ __device__ __forceinline__ void regf_pass1_task(
                     Jz = fma(mr3, fma(al, dz, dvz), Jz);
                 }
                 if constexpr (SCREEN) {
-                    if (any) {
+                    if (__ballot(any) != 0) {
+                        hit.make_room(G);
 #pragma unroll
                         for (int k = 0; k < G; ++k)
                             if (fl[k]) resolve(J[k], jb + k);
@@ -868,6 +878,7 @@ __device__ __forceinline__ void regf_pass1_f64_task(
     double x0 = 0.0, y0 = 0.0, z0 = 0.0, u0 = 0.0, w0 = 0.0, q0 = 0.0;
     double dtr2x = 0.0;   // 2 dtr
     double thr = -1.0;
+    lds.h2[wv][lane] = 0.0;     // read by the lane itself
     if (act) {
         x0 = xi[3 * (size_t)i + 0];
         y0 = xi[3 * (size_t)i + 1];
@@ -876,6 +887,7 @@ __device__ __forceinline__ void regf_pass1_f64_task(
         w0 = vi[3 * (size_t)i + 1];
         q0 = vi[3 * (size_t)i + 2];
         const double h2d = h2[i], dtrd = dtr[i];
+        lds.h2[wv][lane] = h2d;
         dtr2x = 2.0 * dtrd;
         const double chk = x0 + y0 + z0 + u0 + w0 + q0 + h2d + dtrd;
         if (chk != chk) atomicOr(err, ERR_NAN_I);
@@ -933,10 +945,11 @@ __device__ __forceinline__ void regf_pass1_f64_task(
         const double pzd = dz + dtrd * dvz;
         const double r2pd = sq3d(pxd, pyd, pzd);
         const double mnd = r2d < r2pd ? r2d : r2pd;
-        const double h2d = act ? h2[i] : 0.0;   // none past the last i
+        const double h2d = lds.h2[wv][lane];
         const double H = MFLAG ? J.m * h2d : h2d;
         if ((mnd < H) && (j < nj)) {
             hit.push(j);
+            if (hit.n == kHitRows) hit.flush();
         } else if (r2d != 0.0) {
             // Rare (band pairs, r2 < 1e-30): exact FP64 1/sqrt.
             const double rv = fma(dz, dvz, fma(dy, dvy, dx * dvx));
