@@ -86,14 +86,16 @@ __device__ __forceinline__ float pot_run(const PRec *__restrict__ p, double x0,
 
 // As pot_run, on records of which hardly any is at zero distance: without
 // the check first, again with it when a sum is not finite (zero distance:
-// m * inf, or NaN for m = 0).  The check would be 9 of
-// 51 issue cycles a pair.
+// m * inf, or NaN for m = 0).  The check would be 9 of 51 issue cycles a pair.
+// own: the bodies are among the records, so only the run with the check.
 template <bool KEEP, int NJ>
 __device__ __forceinline__ float pot_run_rare(const PRec *__restrict__ p,
                                               double x0, double y0, double z0,
-                                              float a, float *keep) {
-    const float b = pot_run<false, KEEP, NJ>(p, x0, y0, z0, a, keep);
-    if (__ballot(!(fabsf(b) < INFINITY)) == 0) return b;
+                                              float a, float *keep, bool own) {
+    if (!own) {
+        const float b = pot_run<false, KEEP, NJ>(p, x0, y0, z0, a, keep);
+        if (__ballot(!(fabsf(b) < INFINITY)) == 0) return b;
+    }
     return pot_run<true, KEEP, NJ>(p, x0, y0, z0, a, keep);
 }
 
@@ -145,10 +147,16 @@ __global__ __launch_bounds__(64) void k_pot_pass1(const PRec *__restrict__ p,
         y0 = r.y;
         z0 = r.z;
     }
+    // The wavefront's own bodies, b0 and the 63 after it, are in one or two
+    // tiles.  In a call of few tiles a second run of those is its longest task:
+    // 4000 bodies 80 us with it, 73 us so.
+    const int b0 = i0 + iw * 64;
     double A = 0.0;
-    for (int t = tb; t < te; ++t)
+    for (int t = tb; t < te; ++t) {
+        const bool own = (t + 1) * kTile > b0 && t * kTile < b0 + 64;
         A += (double)pot_run_rare<false, kTile>(p + t * kTile, x0, y0, z0, 0.0f,
-                                                nullptr);
+                                                nullptr, own);
+    }
     if (act) part[(size_t)q * nslice + s] = A;
 }
 
@@ -180,9 +188,9 @@ __global__ __launch_bounds__(256) void k_pot_pass2(const double *__restrict__ pa
 // block before its own).
 //
 // Bound: VALU issue, as k_pot_pass1; of its 51 issue cycles a pair, the 43 of
-// the distance and 1/r are paid once for two bodies.  N = 131072: 5.62 ms
-// with a pass over all pairs (2.9e12 pairs/s), 3.4 ms so (2.5e12 unordered
-// pairs/s), the same bits.
+// the distance and 1/r are paid once for two bodies.  N = 131072, the kernel
+// alone: 5.62 ms with a pass over all pairs (3.1e12 pairs/s), 3.4 ms so (2.5e12
+// unordered pairs/s), the same bits.
 // ---------------------------------------------------------------------------
 template <int K>
 __global__ __launch_bounds__(64) void k_pot_sym(const PRec *__restrict__ p,
@@ -233,7 +241,7 @@ __global__ __launch_bounds__(64) void k_pot_sym(const PRec *__restrict__ p,
 #pragma unroll 1
                 for (int h = 0; h < 2; ++h) {
                     a = pot_run_rare<true, kTile / 2>(pj + 32 * h, xi[k], yi[k],
-                                                      zi[k], a, keep + lane);
+                                                      zi[k], a, keep + lane, false);
                     __threadfence_block();
                     if ((lane >> 5) == h) {
                         const float4 *row = reinterpret_cast<const float4 *>(
