@@ -679,10 +679,14 @@ MLP_EXPORT int gpunb_mlp_train(int n, const float *x, const float *t,
         std::mt19937 rng(seed);
         for (int e = 0; e < epochs; ++e) {
             std::shuffle(idx.begin(), idx.end(), rng);
-            // Synchronous, so that idx may be shuffled again; in stream order
+            // Synchronous where idx is shuffled again, and in stream order
             // behind the previous epoch, which reads the old order.
-            MCHK(hipMemcpyWithStream(M.didx, idx.data(), (size_t)n * sizeof(int),
-                                     hipMemcpyHostToDevice, M.st));
+            if (e + 1 < epochs)
+                MCHK(hipMemcpyWithStream(M.didx, idx.data(), (size_t)n * sizeof(int),
+                                         hipMemcpyHostToDevice, M.st));
+            else
+                MCHK(hipMemcpyAsync(M.didx, idx.data(), (size_t)n * sizeof(int),
+                                    hipMemcpyHostToDevice, M.st));
             for (int b = 0; b < nb; ++b) {
                 const int b0 = b * batch;
                 grad_step(std::min(batch, n - b0), b0, M.didx, lr, 1,
