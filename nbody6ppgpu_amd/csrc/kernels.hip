@@ -349,9 +349,10 @@ __global__ void k_zero_int(int *p, int n) {
 // run, the list entries found (row k: entry k of every lane), after them the
 // wavefront's FP64 sums.  Both are kHitRows * 64 ints.  h2: that of the lanes'
 // i for the exact predicate (a register more would cost the mixed kernel a
-// resident wavefront, a load from memory is a wait per flagged pair); 0 for a
-// lane past the last i, which takes no list entry: its position (0, 0, 0) can
-// be a body's, which the mass-weighted screen flags.
+// resident wavefront, a load from memory is a wait per flagged pair: 24
+// clusters of 1000 321 us, 313 so); 0 for a lane past the last i, which takes
+// no list entry: its position (0, 0, 0) can be a body's, which the
+// mass-weighted screen flags.
 constexpr int kHitRows = 14;
 static_assert(kHitRows * 64 * sizeof(int) == 7 * 64 * sizeof(double),
               "the list entries and the sums share a wavefront's LDS");
@@ -385,10 +386,11 @@ struct HitList {
         }
     }
     // Needs room for one more: a full lane is flushed as it fills up (FP64
-    // kernel, scattered i: few lanes of a wavefront have entries at a time), or
-    // room is made for a group of pairs in all lanes together (mixed kernel:
-    // the lanes of nearby i fill up one after the other, and would be flushed
-    // at as many points of the loop).
+    // kernel, scattered i: few lanes of a wavefront have entries at a time;
+    // 4000 i of N = 131072 766 us so, 778 with all lanes at once), or room is
+    // made for a group of pairs in all lanes together (mixed kernel: the lanes
+    // of nearby i fill up one after the other, and would be flushed at as many
+    // points of the loop; all of N = 9000 485 us so, 470 with all at once).
     __device__ __forceinline__ void push(int j) { lds[64 * n++] = j; }
     __device__ __forceinline__ void make_room(int g) {
         if (__ballot(n > kHitRows - g) != 0) flush();
@@ -1027,7 +1029,8 @@ __device__ inline long long xcd_task(long long ntask) {
 // Wavefronts per SIMD that the pass-1 kernels are held to (VGPRs).  At G = 2
 // five fit without spills (the FP64 kernel fits six by itself): King N =
 // 131072, whole step, 14.55 ms at four, 14.3 at five, 14.8 at six (15 VGPRs
-// spilled).  At G = 4 the pair groups need the registers of three.
+// spilled).  The persistent mixed kernel spills six VGPRs at five (24 clusters
+// 2.13 ms, 2.16 at four).  At G = 4 the pair groups need the registers of three.
 constexpr int p1_waves(int g) { return g == 2 ? 5 : 3; }
 
 // Next task of a persistent workgroup.  Tasks [xr[x], xr[x + 1]) belong to
