@@ -93,12 +93,13 @@ constexpr long long kPreMin = 3000000;
 // kMaxBlocks of them at a time; a block of at least kUploadMin bytes is
 // uploaded by the copy engine while the host goes on, a smaller one read from
 // the host by the scatter kernel (8192 bodies, a call: 193 us with the line at
-// 1 MiB, 181 at 512 KiB, 179 at 256 KiB and below).  Of the smaller ones only
-// the first of a kind is a block: each further one would be another scatter
-// launch in the call (1000 bodies in batches of 100: 188 us so, 96 us with the
-// others merged into one block; 6400 in batches of 640: 530 and 495 us).
+// 1 MiB, 181 at 512 KiB, 179 at 256 KiB and below).  Batches past the eighth
+// are merged, as single calls are, into a block of each kind more; as many are
+// kept at rest, or every such call would allocate them again (1000 bodies in
+// batches of 100: 190 us a call with eight kept, 97 so).
 constexpr int kBlockMin = 64;
 constexpr size_t kMaxBlocks = 8;
+constexpr size_t kMaxIdle = kMaxBlocks + 2;
 constexpr size_t kUploadMin = 256 << 10;
 
 // A particle predicted to the call's time: position, velocity, mass.
@@ -330,11 +331,9 @@ struct Block {
     DBuf<char> d;
     const char *src = nullptr;   // where the device reads it
     size_t ints_at() const { return rows ? 0 : (size_t)n * 14 * sizeof(double); }
-    static size_t bytes(bool rows, int n, size_t nflat) {
-        return rows ? (3 * (size_t)n + nflat) * sizeof(int)
-                    : (size_t)n * (14 * sizeof(double) + sizeof(int));
+    size_t bytes() const {
+        return ints_at() + (rows ? 3 * (size_t)n + nflat : (size_t)n) * sizeof(int);
     }
-    size_t bytes() const { return bytes(rows, n, nflat); }
     double *soa() { return (double *)h.p; }
     int *ints() { return (int *)(h.p + ints_at()); }
     void release() {
@@ -519,7 +518,11 @@ Block *take_block(bool rows, int n, size_t nflat) {
     if (!I.idle.empty()) {
         // The one whose buffer fits best: the smallest that is large enough,
         // else the largest.
-        const size_t need = Block::bytes(rows, n, nflat);
+        Block w;
+        w.rows = rows;
+        w.n = n;
+        w.nflat = nflat;
+        const size_t need = w.bytes();
         size_t at = 0;
         for (size_t k = 1; k < I.idle.size(); ++k) {
             const size_t c = I.idle[k]->h.cap, a = I.idle[at]->h.cap;
@@ -584,13 +587,9 @@ void stage_block(bool rows, int n, size_t nflat, F fill) {
     I.blocks.push_back(b);
 }
 
-// Whether a batched call of n bodies, of a block of so many bytes, is staged as
-// a block (lock held).
-bool block_ok(bool rows, int n, size_t bytes) {
+// Whether a batched call of n bodies is staged as a block (lock held).
+bool block_ok(int n) {
     if (n < kBlockMin || I.blocks.size() >= kMaxBlocks) return false;
-    if (bytes < kUploadMin)
-        for (Block *b : I.blocks)
-            if (b->rows == rows) return false;
     if (!I.jp_rec.empty() || !I.ls_hdr.empty()) return false;
     for (Stage *st : g_stages)
         if (st->used.load(std::memory_order_acquire)) return false;
@@ -623,8 +622,7 @@ bool block_jp(int n, const int *addr, const double *x, const double *v,
               const double *f, const double *fd, const double *m,
               const double *t0) {
     std::lock_guard<std::mutex> g(g_stage_mu);
-    if (!block_ok(false, n, Block::bytes(false, n, 0)) || !addresses_once(n, addr))
-        return false;
+    if (!block_ok(n) || !addresses_once(n, addr)) return false;
     stage_block(false, n, 0, [&](Block *b) {
         double *h = b->soa();
         int *slot = b->ints();
@@ -644,15 +642,13 @@ bool block_jp(int n, const int *addr, const double *x, const double *v,
 
 bool block_lists(int n, const int *addr, const int *nnb, const int *members) {
     std::lock_guard<std::mutex> g(g_stage_mu);
-    if (n < kBlockMin) return false;
+    if (!block_ok(n)) return false;
     size_t nf = 0;
     for (int q = 0; q < n; ++q) {
         IREQ(nnb[q] >= 0 && nnb[q] <= I.lstride - 1, "list longer than lmax - 1");
         nf += (size_t)nnb[q];
     }
-    if (nf > (size_t)INT_MAX || !block_ok(true, n, Block::bytes(true, n, nf)) ||
-        !addresses_once(n, addr))
-        return false;
+    if (nf > (size_t)INT_MAX || !addresses_once(n, addr)) return false;
     stage_block(true, n, nf, [&](Block *b) {
         int *hdr = b->ints(), *flat = hdr + 3 * (size_t)n;
         int off = 0;
@@ -942,7 +938,7 @@ void flush_and_force(double t, int ni, const int *addr, double *acc,
     std::lock_guard<std::mutex> g(g_stage_mu);
     for (Block *b : I.blocks) I.idle.push_back(b);
     I.blocks.clear();
-    while (I.idle.size() > kMaxBlocks) {
+    while (I.idle.size() > kMaxIdle) {
         I.idle.back()->release();
         delete I.idle.back();
         I.idle.pop_back();

@@ -23,6 +23,7 @@ size_t most_pinned = SIZE_MAX;   // a larger hipHostMalloc fails
 int fail_uploads = 0;            // that many host-to-device copies fail
 int fail_new = -1;               // operator new fails after so many calls
 size_t held_device = 0;          // bytes of device memory not freed
+int allocations = 0;             // of device and pinned memory
 bool graph_running = false;      // launched, and not waited for since
 int graph_faults = 0;            // executable graphs destroyed while running
 int null_args = 0;               // launches of k_irr_stage without its data
@@ -68,6 +69,7 @@ void stub_most_pinned(size_t bytes) { most_pinned = bytes; }
 void stub_fail_uploads(int n) { fail_uploads = n; }
 void stub_fail_new(int n) { fail_new = n; }
 size_t stub_held_device() { return held_device; }
+int stub_allocations() { return allocations; }
 int stub_graph_faults() { return graph_faults; }
 int stub_null_args() { return null_args; }
 int stub_launches(const char *part) {
@@ -105,6 +107,7 @@ hipError_t hipLaunchKernel(const void *fn, dim3, dim3, void **args, size_t,
 
 hipError_t hipMalloc(void **p, size_t bytes) {
     std::lock_guard<std::mutex> g(mu);
+    ++allocations;
     *p = bytes <= most_device ? take(bytes) : nullptr;
     if (!*p) return last_error = hipErrorOutOfMemory;
     blocks[*p] = bytes;
@@ -122,6 +125,7 @@ hipError_t hipFree(void *p) {
     return hipSuccess;
 }
 hipError_t hipHostMalloc(void **p, size_t bytes, unsigned) {
+    ++allocations;
     *p = bytes <= most_pinned ? take(bytes) : nullptr;
     return *p ? hipSuccess : hipErrorOutOfMemory;
 }

@@ -1,8 +1,8 @@
 """Batches of the irregular force in the order of the calls, where they take
-different ways: large ones (256 KiB and more) are blocks of their own, up to
-eight at a time, of small ones only the first of a kind is.  The last value of a
-body wins, whichever way it came: the forces of 40 bodies against the oracle,
-and the same bits as one batch of the final values."""
+different ways: up to eight are blocks of their own, large ones (256 KiB and
+more) uploaded, small ones read where they are, and the others are merged.  The
+last value of a body wins, whichever way it came: the forces of 40 bodies
+against the oracle, and the same bits as one batch of the final values."""
 import numpy as np
 import pytest
 

@@ -184,19 +184,24 @@ def test_potential_without_memory_for_its_partials(stub):
     """)
 
 
-def test_irr_small_batches_share_scatter_launches(stub):
-    """Ten batches of a hundred bodies, records and lists, and one call: the
-    first batch of each kind and all others together, two launches.  Batches
-    large enough for the copy engine are a launch each."""
+def test_irr_batches_allocate_once(stub):
+    """The same batches again and again, more of them than are blocks of their
+    own, and single calls: no allocation after the first call."""
     run(stub, IRR + """
-    for s in np.split(idx[:1000], 10):
-        jp(s)
-        lists(s)
-    gpunb.irr_firr(0.0, idx[:1000] + 1)
-    assert stub.stub_launches(b"k_irr_stage") == 2
-    for _ in range(3):
+    def call():
+        for s in np.split(idx[:1000], 10):
+            jp(s)
+            lists(s)
         jp(idx)
-    gpunb.irr_firr(0.0, idx[:1000] + 1)
-    assert stub.stub_launches(b"k_irr_stage") == 2 + 3
+        lists(idx)
+        jp(idx[:1])
+        gpunb.irr_firr(0.0, idx[:1000] + 1)
+
+    for _ in range(2):
+        call()
+    before = stub.stub_allocations()
+    for _ in range(3):
+        call()
+    assert stub.stub_allocations() == before
     gpunb.irr_close()
     """)
